@@ -1,27 +1,41 @@
 // Fused backward (stage 1) at four waves per SIMD: bf16 operands, up to 16
-// routes, 2 to 4 taps (the headline layer shape), the work of the fused pass of
-// bwd_tile (moc_mfma.h) on a register budget of 128 VGPRs.
+// routes, 2 to 4 taps (the headline layer shape).
 //
-// Why a second form of the fused pass: the backward is VALU-issue bound, and
-// one SIMD issues fp32 VALU work about 45% faster from four waves than from two
-// (probe on this part: a wave64 v_fma_f32 every 1.7 cycles with four waves per
-// SIMD, 2.5 with two, 5 with one; MFMA and VALU issue do not overlap).  The
-// fused pass of bwd_tile holds 32 channels per wave and needs about 230 VGPRs,
-// i.e. two waves per SIMD.  Here a wave holds 16 channels (one per lane, NC = 1)
-// of the same 32-token super-block, so every per-lane array halves, and a
-// workgroup of 8 waves covers the same 128 channels as bwd_tile's 4: the
-// channel groups, token ranges and partial-sum layouts are those of bwd_tile's
-// grid, and stage 2 is unchanged.
+// What bounds it: instruction issue of four waves per SIMD (a register budget of
+// 128 VGPRs; the two-wave form of bwd_tile, with 32 channels per wave and about
+// 230 VGPRs, issues fp32 work 45% slower).  A wave holds 16 channels, one per
+// lane, and a workgroup of 8 waves the 128 channels of bwd_tile's workgroup, so
+// channel groups, range counts and partial-sum layouts are those of its grid,
+// and stage 2 is the same.
 //
-// Work per super-block and wave (rows t0 .. t0 + 31, own rows the first EOWN):
-//   W_s = alpha . basis_s by MFMA (16x16x16, 16 routes), P = sum_s W_s x_s,
-//   g = dy silu'(P); dx[u] = sum_s g[u+S-1-s] W_s[u+S-1-s] (W at shifted rows
-//   by MFMA on shifted alpha rows, g of the next lane group's first rows by a
-//   cross-lane read); m_s = g x_s split in bf16 hi / lo; dbasis += alpha^T m_s
-//   (16x16x32 over the 32 tokens, accumulated over the whole range in
-//   registers); dalpha += m . basis^T over (tap pair, 16 channels) (16x16x32,
-//   m read back transposed from a wave-private LDS tile with
-//   ds_read_b64_tr_b16); the 8 waves' dalpha tiles summed in LDS in wave order.
+// A range's rows are cut in four streams of 8 n rows, one per 16-lane group of
+// the wave (lane (j, q): channel j, stream q), walked in n steps of 8 rows.  So
+// what a row shares with its neighbours stays in the lane's registers from step
+// to step: the last S - 1 x rows of the window, and the partial dx of the last
+// S - 1 rows, to which later rows still add (dx[t - off] += g[t] W_{S-1-off}[t]:
+// the same W tile that P uses).  A stream hands what its first rows owe to the
+// rows before them to the stream before it through LDS at the end.  Against
+// super-blocks of 32 consecutive rows (three rows of each recomputed in the next,
+// 11 window rows loaded and converted for 8, a second W tile at shifted rows and
+// a cross-lane read of g for dx) a row takes 25% fewer vector instructions and
+// 8 fewer matrix instructions of 32.  B4 T4096 D2048, 16 routes, 4 taps, both
+// stages: with SiLU 92.3 -> 79.9 us (one-element dy 81.8 -> 73.0), D 4096, 32768
+// tokens, no activation 275.0 -> 262.6 us.
+//
+// Work per step and wave (rows 8 i .. 8 i + 7 of each stream):
+//   W_s = alpha . basis_s by MFMA (16x16x16, 16 routes; both operands from LDS,
+//   the basis tile read transposed), P = sum_s W_s x_s, g = dy silu'(P); dx as
+//   above; m_s = g x_s split in bf16 hi / lo; dbasis += alpha^T m_s (16x16x32
+//   over the 32 rows, accumulated over the whole range in registers); dalpha +=
+//   m . basis^T over 16 channels of hi and lo (16x16x32, m read back transposed
+//   from a wave-private LDS tile with ds_read_b64_tr_b16); the 8 waves' dalpha
+//   tiles summed in LDS in wave order.
+//
+// Measured and not kept: x and dy as one 16-byte load per lane through an LDS
+// tile (4x fewer memory instructions, more LDS work: 81.9 us); the rows' scalar
+// offsets in the accesses' soffset (85.8); the next rows fetched before the m
+// products (no change where it fits the registers, 112 us where it spills); the
+// step loop unrolled twice (no change).
 #pragma once
 
 #include "moc_mfma.h"
@@ -64,6 +78,24 @@ constexpr int kLeanCW = 16;        // channels per wave
 // Shapes the lean pass serves (bf16 operands, single launches).
 constexpr bool bwd_lean(int S, int KC, bool bf) { return bf && KC == 1 && S >= 2 && S <= 4; }
 
+// Rows of a row-major tensor walked with the scalar unit: next(bytes) is a buffer
+// from the current row on (`left` bytes; at most 0 past the end: loads give
+// zero, stores drop) and moves `bytes` on.  A lane's byte offset (its stream's
+// first row and its channel) is then the same in every step.  (Opaque after each
+// move: the compiler otherwise precomputes one 64-bit offset per row, more
+// scalars than there are.)
+struct RowWalk {
+  const char* p;
+  int32_t left;
+  __device__ __forceinline__ Buf next(uint32_t bytes, bool on = true) {
+    const Buf b(p, on ? left : 0);
+    p += bytes;
+    left -= static_cast<int32_t>(bytes);
+    asm volatile("" : "+s"(p), "+s"(left));
+    return b;
+  }
+};
+
 // The work of workgroup (bx, by) of one layer; the __global__ wrappers below
 // map a single launch's 2-D grid or a grouped launch's 1-D grid onto it.
 template <int S, int ACT, bool DY1>
@@ -76,26 +108,23 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
   const bool act = ACT == kActRuntime ? act_rt : ACT != 0;  // (uniform)
   using E = uint16_t;
   using Op = s16x4;
-  constexpr int NB = 2, R = 8, TB = 32, W = R + S - 1, EOWN = TB - (S - 1);
-  constexpr int KP = 16, AROWS = TB + S - 1, WPG = kLeanWPG, CW = kLeanCW;
+  constexpr int NB = 2, R = 8, TB = 32, H = S - 1, W = R + H;
+  constexpr int KP = 16, WPG = kLeanWPG, CW = kLeanCW;
   constexpr int ESZ = 2;
   static_assert(S >= 2 && S <= 4, "lean backward: 2 to 4 taps");
 
-  // routing-weight rows of a super-block, twice: copy b holds rows 4 b .. (row
-  // rho of copy b is super-block row rho + 4 b), so that the W operand reads of
-  // token block b at shift e (rows 8 (i / 4) + (i % 4) + e of the copy, e < 4)
-  // never cross an 8-row boundary and sit one immediate apart; unpadded, the
-  // 8-byte chunk c of copy row rho at chunk c ^ ((rho >> 3) & 3) (W operand,
-  // transposed and staging accesses without bank conflicts)
-  constexpr int CROWS = AROWS;
-  __shared__ __align__(16) E a_lds[2][NB][CROWS][KP];
-  __shared__ __align__(16) Op m_tr[WPG][2][2][TrTile1::kSlots];  // [wave][tap of a pair][hi / lo]
+  // routing-weight rows of a step, unpadded: row rho = 8 q + r is row r of
+  // stream q; the 8-byte chunk c (4 routes) of row rho sits at chunk
+  // c ^ ((rho >> 3) & 3) (W operand, transposed and staging accesses without
+  // bank conflicts)
+  __shared__ __align__(16) E a_lds[2][TB][KP];
+  __shared__ __align__(16) Op m_tr[WPG][2][TrTile1::kSlots];  // [wave][hi / lo]
+  // dalpha B operands of each wave, b_lds[wave][s][k = j][4 channels, chunk
+  // q ^ (j / 4)] (a 16-lane group of a read touches 16 distinct slots)
+  __shared__ __align__(16) Op b_lds[WPG][S][16 * 4];
   __shared__ float da_lds[2][WPG][NB][16][17];
-  auto acol = [](int r, int col) -> int { return (col & 3) | (((col >> 2) ^ ((r >> 3) & 3)) << 2); };
+  __shared__ float c0_lds[H][64 * WPG];
 
-  const E* __restrict__ x = static_cast<const E*>(xv);
-  const E* __restrict__ dy = static_cast<const E*>(dyv);
-  E* __restrict__ dx = static_cast<E*>(dxv);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -106,181 +135,214 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
   const int64_t dl = d0 + j;
   const bool ch_ok = wave_on && dl < D;
 
-  // super-blocks [sb_lo, sb_hi) of this range (ranges by < gy1 share the first n_old)
+  // steps [sb_lo, sb_hi) of this range (ranges by < gy1 share the first n_old),
+  // n of them: rows [first, first + 32 n), the last S - 1 not its own
   const int64_t sb_lo = by < gy1 ? static_cast<int64_t>(by) * n_old / gy1
                                  : n_old + static_cast<int64_t>(by - gy1) * (n_total - n_old) / (gy - gy1);
   const int64_t sb_hi = by < gy1 ? static_cast<int64_t>(by + 1) * n_old / gy1
                                  : n_old + static_cast<int64_t>(by + 1 - gy1) * (n_total - n_old) / (gy - gy1);
-  const int nsb = static_cast<int>(sb_hi - sb_lo);
-  const int64_t first = sb_lo * EOWN;
-  const int64_t last_t0 = first + static_cast<int64_t>(nsb - 1) * EOWN;
-  const int64_t row_lo = (first - (S - 1) > 0) ? first - (S - 1) : 0;
-  const int64_t row_hi = (last_t0 + TB < N) ? last_t0 + TB : N;
-  const int64_t a_hi = (last_t0 + AROWS < N) ? last_t0 + AROWS : N;
+  const int n = static_cast<int>(sb_hi - sb_lo);
+  const int64_t first = sb_lo * TB - static_cast<int64_t>(by) * H;
+  const int64_t end = first + static_cast<int64_t>(n) * TB;
+  const int64_t row_hi = end < N ? end : N;            // rows read
+  const int64_t own_hi = end - H < N ? end - H : N;    // rows owned
+  const int srow = R * n * q;                          // first row of this lane's stream
   const uint32_t rb = static_cast<uint32_t>(D * ESZ);
   const uint32_t col = static_cast<uint32_t>(dl * ESZ);
-  const Buf xb(x + row_lo * D, (row_hi - row_lo) * D * ESZ);
+  const uint32_t vx = ch_ok ? static_cast<uint32_t>(srow) * rb + col : kOffNone;
+  RowWalk xwalk{static_cast<const char*>(xv) + first * rb, static_cast<int32_t>((row_hi - first) * rb)};
+  RowWalk dxw{static_cast<const char*>(dxv) + (first - H) * rb,
+              static_cast<int32_t>((own_hi - first + H) * rb)};
   // dy rows dys elements apart (D; 0: one row for all tokens; -1: one element
-  // for every token and channel, the expanded gradient of a sum to a scalar).
-  // DY1 (dys = -1 in every layer of the launch): the element is read once here,
-  // no row loads and no conversions in the loop.  Otherwise a -1 of one layer
-  // is served by OR-ing the element's fp32 bits into every converted dy value
-  // while the row loads read nothing (no branch in the loop)
+  // for every token and channel, the expanded gradient of a sum).  DY1 (dys =
+  // -1 in every layer of the launch): the element is read once.  Otherwise a -1
+  // of one layer reads the element in place of every row (rows 0 bytes apart,
+  // no channel offset)
   const bool dy_one = DY1 || dys < 0;
   const uint32_t drb = static_cast<uint32_t>((dy_one ? 0 : dys) * ESZ);
-  const Buf dyb(dy_one ? dy : dy + row_lo * dys, dy_one ? ESZ : ((row_hi - row_lo - 1) * dys + D) * ESZ);
-  uint32_t dy_or = 0;
-  if (dy_one) {
+  const uint32_t vdy = ch_ok ? static_cast<uint32_t>(srow) * drb + (dy_one ? 0u : col) : kOffNone;
+  // (the bytes after row w: rows up to row_hi, the last one D elements long)
+  RowWalk dyw{static_cast<const char*>(dyv) + first * drb,
+              static_cast<int32_t>(dy_one ? ESZ
+                                          : (row_hi > first ? (row_hi - first - 1) * drb + D * ESZ : 0))};
+  float dy1 = 0.f;
+  if constexpr (DY1) {
     E e;
-    dyb.load<ESZ>(0, &e);
-    dy_or = ch_ok ? __float_as_uint(bf16_to_f32(e)) : 0u;
+    Buf(dyv, ESZ).load<ESZ>(ch_ok ? 0u : kOffNone, &e);
+    dy1 = bf16_to_f32(e);
   }
-  const bool dy_rows = ch_ok && !dy_one;
-  const Buf ab(a_c + first * KP, (a_hi - first) * KP * ESZ);
   const Buf bb(b_c, static_cast<int64_t>(KP) * S * D * ESZ);
 
-  // W operands: bop[s] = basis[4 q + v, s, dl] (B operand, column = this lane's channel)
-  Op bop[S];
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    E e[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) bb.load<ESZ>(row_off((4 * q + v) * S + s, 0, rb, col, ch_ok), &e[v]);
-    bop[s] = CT<true>::make(e[0], e[1], e[2], e[3]);
-  }
-  // dalpha B operands: bda[s] = basis[j, s, d0 + 4 q + {0..3}] (channels past D,
+  // dalpha B operands: basis[j, s, d0 + 4 q + {0..3}] (channels past D,
   // with D % 4 == 2 the last two of the final group, zero: the load reaches into
   // the next row)
-  Op bda[S];
   {
     const int64_t ch = d0 + 4 * q;
     const bool on = wave_on && ch < D;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-      bb.load<8>(row_off(j * S + s, 0, rb, static_cast<uint32_t>(ch * ESZ), on), &bda[s]);
+      Op bda;
+      bb.load<8>(row_off(j * S + s, 0, rb, static_cast<uint32_t>(ch * ESZ), on), &bda);
       if (ch + 2 >= D) {
-        bda[s][2] = 0;
-        bda[s][3] = 0;
+        bda[2] = 0;
+        bda[3] = 0;
       }
+      b_lds[wave][s][j * 4 + (q ^ (j >> 2))] = bda;
     }
   }
   f32x4 dbacc[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) dbacc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // raw rows of one super-block: x window (trun - (S-1) .. trun + R - 1), dy rows
-  E xr[W], dr[DY1 ? 1 : R];
-  auto fetch_xdy = [&](int64_t t0) {
-    const uint32_t base = row_off(t0 + R * q - (S - 1), row_lo, rb, col, ch_ok);
+  // raw rows of one step
+  E xr[R], dr[DY1 ? 1 : R];
+  // (two rows per buffer: one more vector add against six scalar instructions)
+  auto fetch_xdy = [&]() {
 #pragma unroll
-    for (int w = 0; w < W; ++w) xb.load<ESZ>(base + w * rb, &xr[w]);
+    for (int r = 0; r < R; r += 2) {
+      const Buf b = xwalk.next(2 * rb);
+      b.load<ESZ>(vx, &xr[r]);
+      b.load<ESZ>(vx + rb, &xr[r + 1]);
+    }
     if constexpr (!DY1) {
-      const uint32_t dbase = row_off(t0 + R * q, row_lo, drb, col, dy_rows);
 #pragma unroll
-      for (int r = 0; r < R; ++r) dyb.load<ESZ>(dbase + r * drb, &dr[r]);
+      for (int r = 0; r < R; r += 2) {
+        const Buf b = dyw.next(2 * drb);
+        b.load<ESZ>(vdy, &dr[r]);
+        b.load<ESZ>(vdy + drb, &dr[r + 1]);
+      }
     }
   };
-  // routing-weight rows of a super-block: AROWS x 16 elements, 8 bytes per thread
-  constexpr int ACHUNKS = AROWS * KP / 4;
-  static_assert(ACHUNKS <= 64 * WPG, "one routing-weight chunk per thread");
-  E arw[4];
+  // routing-weight rows of a step: 32 x 16 elements, 8 bytes per thread of the
+  // first two waves (row rho: thread rho 4 + chunk)
   // (the per-lane terms are formed where they are used, from an opaque copy of
-  // the thread id: hoisted out of the loop they outgrew the register budget)
+  // the thread id: hoisted out of the loop they outgrow the register budget)
   auto opaque_tid = [&]() {
     int t = tid;
     asm volatile("" : "+v"(t));
     return t;
   };
-  auto fetch_a = [&](int64_t t0) {
-    const int tt = opaque_tid();
-    ab.load<8>(row_off(t0 + (tt >> 2), first, KP * ESZ, (tt & 3) * 8, tt < ACHUNKS), arw);
+  static_assert(TB * KP / 4 == 128, "two waves fetch a step's routing weights");
+  RowWalk aw{reinterpret_cast<const char*>(a_c + first * KP), static_cast<int32_t>((row_hi - first) * KP * ESZ)};
+  E arw[4];
+  auto fetch_a = [&]() {
+    const Buf ab = aw.next(R * KP * ESZ);
+    if (wave < 2) {
+      const int t = opaque_tid(), row = t >> 2;
+      ab.load<8>(static_cast<uint32_t>((R * n * (row >> 3) + (row & 7)) * KP * ESZ + (t & 3) * 8), arw);
+    }
   };
   auto stage_alpha = [&](int buf) {
-    const int tt = opaque_tid();
-    const int row = tt >> 2, c4 = (tt & 3) * 4;
-    if (tt < ACHUNKS) {
-      Vec<E, 4>::store(&a_lds[buf][0][row][acol(row, c4)], arw);
-      if (row >= 4) Vec<E, 4>::store(&a_lds[buf][1][row - 4][acol(row - 4, c4)], arw);
+    if (wave < 2) {
+      const int t = opaque_tid(), row = t >> 2;
+      Vec<E, 4>::store(&a_lds[buf][row][((t & 3) ^ ((row >> 3) & 3)) * 4], arw);
     }
   };
 
-  if (first < N) {
-    fetch_xdy(first);
-    fetch_a(first);
-    stage_alpha(0);
+  // the window rows before the stream: rows first + srow - H + w
+  float xw[W];
+#pragma unroll
+  for (int w = 0; w < H; ++w) {
+    const int64_t u = first + srow - H + w;
+    E e;
+    const int64_t lo = first - H > 0 ? first - H : 0;
+    Buf(static_cast<const char*>(xv) + lo * rb, (row_hi - lo) * rb).load<ESZ>(row_off(u, lo, rb, col, ch_ok), &e);
+    xw[R + w] = bf16_to_f32(e);
   }
+  fetch_xdy();
+  fetch_a();
+  stage_alpha(0);
   __syncthreads();
 
-  StartCursor cursor;
-  // dalpha partials of this channel group from row `first` on (rows
-  // [first, row_hi), 16 routes; 32-bit offsets within the range)
-  const Buf pdab(part_da + (static_cast<int64_t>(bx) * N + first) * KP, (row_hi - first) * KP * 4);
-  for (int sb = 0; sb < nsb; ++sb) {
-    const int64_t t0 = first + static_cast<int64_t>(sb) * EOWN;
-    if (t0 >= N) break;  // uniform over the workgroup
-    const int buf = sb & 1;
-    const int64_t own_end = (t0 + EOWN < N) ? t0 + EOWN : N;
-    // the lane's terms formed here each time (see opaque_tid); they shadow the
-    // function-scope ones in the loop body
+  // the next segment start at or after this lane's window (rows from `first`;
+  // the token axis's end counts as one), searched again once a window passed it
+  const int32_t n_rel = static_cast<int32_t>(N - first < (int64_t(1) << 30) ? N - first : int64_t(1) << 30);
+  auto start_from = [&](int64_t rel) -> int32_t {
+    const int64_t st = seq.next_start(first + rel) - first;
+    return static_cast<int32_t>(st < n_rel ? st : n_rel);
+  };
+  int32_t ns = start_from(srow - (S - 2));
+
+  // dx rows -(S-1) .. R-1 of a step: dxa[w] is row w - (S-1); the first S-1 carry
+  // over from the step before.  c0_lds: what a stream's first rows add to the
+  // rows before it, which the stream before takes at the end
+  float dxa[W];
+#pragma unroll
+  for (int e = 0; e < H; ++e) dxa[R + e] = 0.f;
+
+  // dalpha partials of this channel group from row `first` on (own rows, 16 routes)
+  RowWalk pdw{reinterpret_cast<const char*>(part_da + (static_cast<int64_t>(bx) * N + first) * KP),
+              static_cast<int32_t>((own_hi - first) * KP * 4)};
+
+  auto step = [&](int i, auto mask_tag) {
+    constexpr bool MASK = decltype(mask_tag)::value;
     const int tl = opaque_tid();
-    const int lane = tl & 63;
-    const int j = lane & 15, q = lane >> 4;
-    const int64_t trun = t0 + R * q;
-    const bool more = (sb + 1 < nsb) && (t0 + EOWN < N);
-
-    float xw[W], g[R];
+    const int j = tl & 15, q = (tl >> 4) & 3;
+    const int buf = i & 1;
+    const bool more = i + 1 < n;
 #pragma unroll
-    for (int w = 0; w < W; ++w) xw[w] = bf16_to_f32(xr[w]);
+    for (int w = 0; w < H; ++w) {
+      xw[w] = xw[R + w];
+      dxa[w] = dxa[R + w];
+    }
+    float g[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-      g[r] = DY1 ? __uint_as_float(dy_or) : __uint_as_float(__float_as_uint(bf16_to_f32(dr[DY1 ? 0 : r])) | dy_or);
-    // the next super-block's routing weights (unconditionally: after the last
-    // super-block of the range they fall past the buffer and load zeros, and
-    // the rows just converted are dead, so the loop carries no copies)
-    fetch_a(t0 + EOWN);
+    for (int r = 0; r < R; ++r) {
+      xw[H + r] = bf16_to_f32(xr[r]);
+      g[r] = DY1 ? dy1 : bf16_to_f32(dr[DY1 ? 0 : r]);
+    }
+    // (unconditionally, also after the last step: rows past the buffer load zeros)
+    fetch_a();
 
-    // alpha operand of token block b shifted by e < 4 rows (row i = j): row
-    // r = R (j / 4) + j % 4 + e of copy b, chunk q ^ (r >> 3) = q ^ (j / 4)
-    // (j % 4 + e < 8): one lane offset plus immediates
-    const char* a_base = reinterpret_cast<const char*>(&a_lds[buf][0][0][0]) +
-                         ((R * (j >> 2) + (j & 3)) * KP + ((q ^ (j >> 2)) << 2)) * ESZ;
-    auto aop = [&](int e, int b) -> Op {
-      return *reinterpret_cast<const Op*>(a_base + ((b * CROWS + e) * KP) * ESZ);
-    };
-
-    const int64_t w_lo = t0 - (S - 2), w_hi = t0 + TB + S - 2;
-    const bool interior = !cursor.starts_in(seq, w_lo, w_hi);
+    // alpha operand of token block b: row 8 (j / 4) + 4 b + j % 4, chunk q ^ (j / 4)
+    Op aop[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      aop[b] = *reinterpret_cast<const Op*>(&a_lds[buf][R * (j >> 2) + 4 * b + (j & 3)][(q ^ (j >> 2)) * 4]);
 
     f32x4 dacc[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b) dacc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    auto body = [&](auto mask_tag) {
-      constexpr bool MASK = decltype(mask_tag)::value;
-      // masks of this lane's run extended by S-1 later rows (rows r < R + S - 1),
-      // packed in two registers: bit k of `sb` is set when window row
-      // trun - (S-1) + k starts a segment, bit r of `rv` when row trun + r is a
-      // token (< N); tap s of row r is valid when the row is a token and no
-      // segment starts in window rows r + s + 1 .. r + S - 1
+    {
+      // bit k of `sbm`: window row t0 - (S-1) + k starts a segment; bit r of
+      // `rv`: row t0 + r is a token (< N); tap s of row r is valid when the row
+      // is a token and no segment starts in window rows r + s + 1 .. r + S - 1
       uint32_t sbm = 0, rv = 0;
       if constexpr (MASK) {
-        const int64_t u0 = trun - (S - 1);
-        for (int64_t st = seq.next_start(w_lo); st <= w_hi && st < N; st = seq.next_start(st + 1)) {
-          const int64_t k = st - u0;
-          if (k > 0 && k < 32) sbm |= 1u << k;
+        const int32_t t0 = R * n * q + R * i;  // this lane's first row (from `first`)
+        const int32_t u0 = t0 - H, lo_next = t0 + R - (S - 2);
+        int32_t st = ns;
+        while (st <= t0 + R - 1 && st < n_rel) {
+          const int32_t k = st - u0;
+          if (k > 0) sbm |= 1u << k;
+          const int32_t nx = start_from(static_cast<int64_t>(st) + 1);
+          if (st < lo_next) ns = nx;
+          st = nx;
         }
-        const int64_t nrow = N - trun;  // rows r < nrow are tokens
-        rv = nrow >= 32 ? ~0u : (nrow <= 0 ? 0u : ((1u << nrow) - 1u));
+        const int32_t nrow = n_rel - t0;  // rows r < nrow are tokens
+        rv = nrow >= R ? 0xffu : (nrow <= 0 ? 0u : ((1u << nrow) - 1u));
       }
       auto tap_ok = [&](int r, int s) -> bool {
         if constexpr (MASK) {
-          constexpr uint32_t kNone = 0;
           const uint32_t span = ((1u << (S - 1 - s)) - 1u) << (r + s + 1);
-          return ((rv >> r) & 1u) && (sbm & span) == kNone;
+          return ((rv >> r) & 1u) && (sbm & span) == 0;
         } else {
           return true;
         }
       };
+
+      // basis[4 q + v, s, channel j]: the tile's rows read transposed
+      Op bop[S];
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+        bop[s] = TrTile<NB, 2>::read(&b_lds[wave][s][(4 * q + (j >> 2)) * 4 + ((j & 3) ^ q)]);
+      // W of this lane's rows: P and dx both read it
+      f32x4 w4[S][NB];
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) w4[s][b] = mma16(aop[b], bop[s], f32x4{0.f, 0.f, 0.f, 0.f});
 
       if constexpr (ACT != 0) if (act) {  // (act: uniform; always with a fixed ACT)
         float p[R];
@@ -289,14 +351,8 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
 #pragma unroll
         for (int s = 0; s < S; ++s)
 #pragma unroll
-          for (int b = 0; b < NB; ++b) {
-            const f32x4 w4 = mma16(aop(0, b), bop[s], f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              const int r = 4 * b + v;
-              if (tap_ok(r, s)) p[r] = fmaf(xw[r + s], w4[v], p[r]);
-            }
-          }
+          for (int r = 0; r < R; ++r)
+            if (tap_ok(r, s)) p[r] = fmaf(xw[r + s], w4[s][r >> 2][r & 3], p[r]);
         // g *= silu'(P) = sg (1 + P (1 - sg)), sg = sigmoid(P) as sigmoid_f forms it
         float sg[R];
 #pragma unroll
@@ -310,64 +366,44 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
         }
       }
 
-      // dx, taps in descending order (the first need none of the next lane
-      // group's rows)
-      if (dx != nullptr) {
-        float gf[S - 1];
-        const int src_lane = (lane + 16) & 63;
+      // dx[t - off] += g[t] W_{S-1-off}[t], nearest rows first
+      if (dxv != nullptr) {
 #pragma unroll
-        for (int e = 0; e < S - 1; ++e) gf[e] = __shfl(g[e], src_lane, 64);
-        float dxa[R];
+        for (int r = 0; r < R; ++r) dxa[H + r] = 0.f;
 #pragma unroll
-        for (int r = 0; r < R; ++r) dxa[r] = 0.f;
+        for (int off = 0; off < S; ++off)
 #pragma unroll
-        for (int si = 0; si < S; ++si) {
-          const int s = S - 1 - si, off = S - 1 - s;
+          for (int r = 0; r < R; ++r)
+            if (tap_ok(r, S - 1 - off))
+              dxa[H + r - off] = fmaf(g[r], w4[S - 1 - off][r >> 2][r & 3], dxa[H + r - off]);
+        if (i == 0) {
 #pragma unroll
-          for (int b = 0; b < NB; ++b) {
-            const f32x4 w4 = mma16(aop(off, b), bop[s], f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              const int r = 4 * b + v, src = r + off;
-              const float gs = (src < R) ? g[src < R ? src : 0] : gf[src >= R ? src - R : 0];
-              if (tap_ok(src, s)) dxa[r] = fmaf(gs, w4[v], dxa[r]);
-            }
-          }
+          for (int e = 0; e < H; ++e) c0_lds[e][tl] = dxa[e];
         }
-        // the buffer ends at this super-block's last own row: later rows drop
-        const Buf dxb(dx + row_lo * D, (own_end - row_lo) * D * ESZ);
-        const uint32_t base = row_off(trun, row_lo, rb, col, ch_ok);
+        // rows -(S-1) .. R-S of the step are complete; before the first step's
+        // they belong to the stream (or range) before
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const E o = f32_to_bf16(dxa[r]);
-          dxb.store<ESZ>(base + r * rb, &o);
+        for (int w = 0; w < R; ++w) {
+          const E o = f32_to_bf16(dxa[w]);
+          dxw.next(rb, w >= H || i > 0).store<ESZ>(vx, &o);
         }
       }
 
-      // alpha^T operands of the dbasis MFMA, own rows only:
-      // at[b] = alpha[trun + 4 b + v, j] (transposed read of the staged rows)
+      // alpha^T operands of the dbasis MFMA, own rows only (the last step's
+      // final S-1 rows of stream 3 are the next range's; rows past N are zero):
+      // at[b] = alpha[row 8 q + 4 b + v, j] (transposed read of the staged rows)
       Op at[NB];
-      {
-        const int own_rows = static_cast<int>(own_end - t0);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          uint64_t keep;
-          if (own_rows == EOWN) {
-            // (uniform) every super-block but the token axis's last: rows
-            // R q + 4 b + v < EOWN hold for all but the last block of group 3,
-            // which keeps its first EOWN - (TB - 4) rows
-            keep = (b == NB - 1 && q == 3) ? ((1ull << (16 * (EOWN - (TB - 4)))) - 1ull) : ~0ull;
-          } else {
-            const int n_ok = min(max(own_rows - (R * q + 4 * b), 0), 4);
-            keep = n_ok >= 4 ? ~0ull : ((1ull << (16 * n_ok)) - 1ull);
-          }
-          const int r = R * q + 4 * b + (j >> 2);
-          const Op v = TrTile<NB, 2>::read(&a_lds[buf][0][r][acol(r, 4 * (j & 3))]);
-          at[b] = __builtin_bit_cast(Op, __builtin_bit_cast(uint64_t, v) & keep);
-        }
+      for (int b = 0; b < NB; ++b) {
+        const int r = R * q + 4 * b + (j >> 2);
+        at[b] = TrTile<NB, 2>::read(&a_lds[buf][r][((j & 3) ^ q) * 4]);
       }
-      // m of tap s -> hi / lo operands -> this wave's tile slot p, dbasis MFMAs
-      auto stage_m = [&](int s, int p) {
+      if (!more) {
+        const uint64_t keep = q == 3 ? ((1ull << (16 * (4 - H))) - 1ull) : ~0ull;
+        at[NB - 1] = __builtin_bit_cast(Op, __builtin_bit_cast(uint64_t, at[NB - 1]) & keep);
+      }
+      // m of tap s -> hi / lo operands -> this wave's tile, dbasis MFMAs
+      auto stage_m = [&](int s) {
         Op mh[NB], ml[NB];
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
@@ -382,58 +418,39 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
           }
           mh[b] = pack4_hi(hbits[0], hbits[1], hbits[2], hbits[3]);
           ml[b] = pack4_bf16(lo[0], lo[1], lo[2], lo[3]);
-          m_tr[wave][p][0][TrTile1::wslot(j, q, b)] = mh[b];
-          m_tr[wave][p][1][TrTile1::wslot(j, q, b)] = ml[b];
+          m_tr[wave][0][TrTile1::wslot(j, q, b)] = mh[b];
+          m_tr[wave][1][TrTile1::wslot(j, q, b)] = ml[b];
         }
         dbacc[s] = mma32(mh[0], mh[1], at[0], at[1], dbacc[s]);
         dbacc[s] = mma32(ml[0], ml[1], at[0], at[1], dbacc[s]);
       };
-      // transposed reads of tile slot p: ra[rb][h] = m[16 rb + i][4 qq + {0..3}]
-      auto read_m = [&](int p, Op (&ra)[NB][2]) {
+      // dalpha contracts 16 channels of the hi and of the lo part in one
+      // 16x16x32 MFMA against the basis operand twice.  The transposed reads of
+      // a tap (ra[rb][h] = m[16 rb + i][4 qq + {0..3}]) are issued before the next
+      // tap's m values are formed and written (a wave's LDS operations complete
+      // in issue order, so one tile serves)
+      Op ra[NB][2], bda;
+      stage_m(0);
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        wave_lds_sync();
 #pragma unroll
         for (int r2 = 0; r2 < NB; ++r2)
 #pragma unroll
           for (int h = 0; h < 2; ++h)
-            ra[r2][h] = TrTile<NB, 2>::read(&m_tr[wave][p][h][TrTile1::rslot(j, q, r2)]);
-      };
-      // tap pairs (s, s + 1): dalpha contracts (tap, 16 channels) pairs in one
-      // 16x16x32 MFMA; an odd last tap alone in a 16x16x16 one.  The reads of a
-      // pair are issued before the next pair's m values are formed and written
-      // (a wave's LDS operations complete in issue order, so one tile serves).
-      constexpr int NPAIR = (S + 1) / 2;
-      Op ra0[NB][2], ra1[NB][2];
-#pragma unroll
-      for (int pi = 0; pi < NPAIR; ++pi) {
-        const int s0 = 2 * pi;
-        const bool two = s0 + 1 < S;
-        if (pi == 0) {
-          stage_m(s0, 0);
-          if (two) stage_m(s0 + 1, 1);
-        }
-        wave_lds_sync();
-        read_m(0, ra0);
-        if (two) read_m(1, ra1);
+            ra[r2][h] = TrTile<NB, 2>::read(&m_tr[wave][h][TrTile1::rslot(j, q, r2)]);
+        bda = b_lds[wave][s][j * 4 + (q ^ (j >> 2))];
         __builtin_amdgcn_sched_barrier(0);
-        if (pi + 1 < NPAIR) {
-          stage_m(s0 + 2, 0);
-          if (s0 + 3 < S) stage_m(s0 + 3, 1);
-        }
+        if (s + 1 < S) stage_m(s + 1);
 #pragma unroll
-        for (int r2 = 0; r2 < NB; ++r2)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            if (two) dacc[r2] = mma32(ra0[r2][h], ra1[r2][h], bda[s0], bda[two ? s0 + 1 : s0], dacc[r2]);
-            else dacc[r2] = mma16(ra0[r2][h], bda[s0], dacc[r2]);
-          }
+        for (int r2 = 0; r2 < NB; ++r2) dacc[r2] = mma32(ra[r2][0], ra[r2][1], bda, bda, dacc[r2]);
       }
       wave_lds_sync();
-    };
-    if (interior) body(std::false_type{});
-    else body(std::true_type{});
-    // the next super-block's rows, into the registers the raw rows left
+    }
+    // the next step's rows, into the registers the raw rows left
     // (unconditionally, as fetch_a above); issued after the m products, where
     // the fewest registers are live, and covered by the other waves of the SIMD
-    fetch_xdy(t0 + EOWN);
+    fetch_xdy();
 
 #pragma unroll
     for (int r2 = 0; r2 < NB; ++r2)
@@ -441,7 +458,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
       for (int v = 0; v < 4; ++v) da_lds[buf][wave][r2][4 * q + v][j] = dacc[r2][v];
     if (more) stage_alpha(buf ^ 1);
     __syncthreads();
-    // sum the 8 waves' dalpha tiles in wave order; own rows only
+    // sum the 8 waves' dalpha tiles in wave order; rows past the own ones drop
     {
       const int r2 = tl >> 8, row = (tl >> 4) & 15, c = tl & 15;
       float tv[WPG];
@@ -450,9 +467,26 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
       float sum = 0.f;
 #pragma unroll
       for (int w = 0; w < WPG; ++w) sum += tv[w];
-      const int n_own = static_cast<int>(own_end - t0);
-      const uint32_t off = static_cast<uint32_t>(((t0 - first + 16 * r2 + row) * KP + c) * 4);
-      pdab.store<4>(16 * r2 + row < n_own ? off : kOffNone, &sum);
+      const int rho = tl >> 4;
+      pdw.next(R * KP * 4)
+          .store<4>(static_cast<uint32_t>(((R * n * (rho >> 3) + (rho & 7)) * KP + c) * 4), &sum);
+    }
+  };
+  // plain steps in a loop of their own: the accumulators stay in their registers
+  // there (with both forms joined in one loop body they were moved every step)
+  for (int i = 0; i < n; ++i) {
+    for (; i < n && __builtin_amdgcn_ballot_w64(ns <= srow + R * i + R - 1) == 0; ++i)
+      step(i, std::false_type{});
+    if (i < n) step(i, std::true_type{});
+  }
+
+  // the last S-1 rows of a stream: what its own rows gave them, and what the next
+  // stream's first rows did (stream 3's are past the own rows and drop)
+  if (dxv != nullptr) {
+#pragma unroll
+    for (int e = 0; e < H; ++e) {
+      const E o = f32_to_bf16(dxa[R + e] + c0_lds[e][(tid & ~63) | ((lane + 16) & 63)]);
+      dxw.next(rb).store<ESZ>(vx, &o);
     }
   }
 

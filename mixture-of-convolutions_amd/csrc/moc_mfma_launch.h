@@ -178,6 +178,26 @@ inline Grid2 bwd_grid_tiered(int64_t N, int64_t gx, int64_t D, int64_t S, int n_
   return g;
 }
 
+// Grid of the lean fused pass (moc_bwd_lean.h): the channel groups, range count
+// and tiers above, but counted in steps of 32 rows of which a range gives up
+// S - 1 in all (n steps own 32 n - (S - 1) rows; range by starts at row
+// 32 steps_before - by (S - 1)).  Every range has at least one step: there are
+// at most ceil(N / (32 - (S - 1))) ranges.
+inline Grid2 bwd_lean_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int n_cu) {
+  Grid2 g = bwd_grid_tiered(N, gx, D, S, n_cu);
+  const int64_t gy = g.gy, gy1 = g.gy1;
+  const int64_t steps = cdiv(N + gy * (S - 1), 16 * kBwdNB);
+  const int64_t n_old = (steps * kBwdOldShare + 50) / 100;
+  if (gy1 < gy && n_old >= gy1 && steps - n_old >= gy - gy1) {
+    g.n_old = static_cast<int>(n_old);
+  } else {
+    g.gy1 = static_cast<int>(gy);
+    g.n_old = static_cast<int>(steps);
+  }
+  g.n_total = static_cast<int>(steps);
+  return g;
+}
+
 // The backward in two passes (bwd_kernel modes kBwdDx, then kBwdTaps with the
 // taps split in halves) where the fused pass does not fit two waves per SIMD
 // and no activation needs P: bf16, 32 routes and 4 to 8 taps, 16 routes and 7
@@ -298,8 +318,9 @@ void bwd_one(const Problem& p, const void* x, const void* dy, const void* a_c, c
   // tiers for the fused pass at two resident workgroups per CU (not split in route chunks)
   constexpr bool kTiers = !kTwo && !kSplit && kBwdMinWaves<S, KC, kBwdFused, BF> == 2;
   const int64_t gx_all = cdiv(p.D, kBwdCW);
-  const Grid2 g = kTiers ? bwd_grid_tiered(p.n_tokens, gx_all, p.D, S, device_cu_count())
-                         : bwd_grid(p.n_tokens, p.D, S);
+  const Grid2 g = kLean    ? bwd_lean_grid(p.n_tokens, gx_all, p.D, S, device_cu_count())
+                  : kTiers ? bwd_grid_tiered(p.n_tokens, gx_all, p.D, S, device_cu_count())
+                           : bwd_grid(p.n_tokens, p.D, S);
   const auto* a = static_cast<const E*>(a_c);
   const auto* b = static_cast<const E*>(b_c);
   const int gx = static_cast<int>(g.gx), gy = static_cast<int>(g.gy);
@@ -383,6 +404,7 @@ void bwd_layers_one(const Problem& p, const LayerOps* L, int n, hipStream_t st) 
                                       bwd_two_pass_r(S, KC, false, true))) ||
                         kTwoG;
   constexpr int kParts = kTwo ? taps_route_parts(KC) : 1;
+  constexpr bool kLean = MOC_BWD_LEAN && !kTwo && bwd_lean(S, KC, true);
   constexpr bool kTiers = !kTwo && !kSplit && kBwdMinWaves<S, KC, kBwdFused, true> == 2;
   const int n_cu = device_cu_count();
   // each layer's grid as bwd_one forms it (the taps pass has its own)
@@ -392,8 +414,9 @@ void bwd_layers_one(const Problem& p, const LayerOps* L, int n, hipStream_t st) 
   bool any_dx = false;
   for (int i = 0; i < n; ++i) {
     const int64_t gx_l = cdiv(L[i].D, kBwdCW);
-    const Grid2 g = kTiers ? bwd_grid_tiered(p.n_tokens, gx_l, L[i].D, S, n_cu)
-                           : bwd_grid(p.n_tokens, L[i].D, S);
+    const Grid2 g = kLean    ? bwd_lean_grid(p.n_tokens, gx_l, L[i].D, S, n_cu)
+                    : kTiers ? bwd_grid_tiered(p.n_tokens, gx_l, L[i].D, S, n_cu)
+                             : bwd_grid(p.n_tokens, L[i].D, S);
     ly.l[i] = BwdLayer{L[i].x, L[i].dy, L[i].dys, L[i].a_c, L[i].b_c, L[i].dx, L[i].part_da,
                        L[i].part_db, L[i].D, static_cast<int>(g.gx), static_cast<int>(g.gy),
                        g.gy1, g.n_old, g.n_total, static_cast<int>(blk), L[i].act,
@@ -425,7 +448,7 @@ void bwd_layers_one(const Problem& p, const LayerOps* L, int n, hipStream_t st) 
                          dim3(static_cast<unsigned>(blk)), dim3(64 * kBwdWPG), 0, st, ly, p.seq);
     hipLaunchKernelGGL((bwd_layers_kernel<S, KC, kBwdNB, kBwdNC, kTapsWPG, ACT, true, (kParts > 1), kBwdTaps>),
                        dim3(static_cast<unsigned>(blkt)), dim3(64 * kTapsWPG), 0, st, lt, p.seq);
-  } else if constexpr (MOC_BWD_LEAN && bwd_lean(S, KC, true)) {
+  } else if constexpr (kLean) {
     // (layers whose dy is one element each, or none of them: one instantiation
     // per form; mixed forms keep every layer's rows by the general one)
     bool all_one = true;

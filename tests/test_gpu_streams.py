@@ -1,0 +1,66 @@
+"""The stream form of the fused backward (2 to 4 taps, up to 16 routes, bf16):
+ranges of one and of several steps, token counts around a step and a range, a
+ragged last channel group, segment starts at every place of a stream (between
+streams, steps and ranges included), against the oracle."""
+import pytest
+import torch
+
+from moc import moc_triton
+from oracle import moc_oracle as O
+from tests._parity import assert_close, gen, randn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+BF = torch.bfloat16
+
+
+def _check(x, a, b, dy, act, lengths=None):
+    xx, aa, bb = (t.to(DEV, BF).requires_grad_() for t in (x, a, b))
+    if lengths is None:
+        y, _ = moc_triton(xx, aa, bb, activation=act)
+    else:
+        cu = torch.tensor([0, *lengths]).cumsum(0).to(DEV, torch.int32)
+        y, _ = moc_triton(xx, aa, bb, activation=act, cu_seqlens=cu, max_seqlen=max(lengths))
+    y.backward(dy.to(DEV, BF).expand_as(y))
+    rx, ra, rb = (t.detach().clone().requires_grad_() for t in O.reference_inputs(x.to(BF), a.to(BF), b.to(BF), BF))
+    if lengths is None:
+        ry = O.moc_ref(rx, ra, rb, act)
+    else:
+        ry = O.moc_varlen_ref(rx, ra, rb, cu.cpu(), act)
+    ry.backward(dy.to(BF).float().expand_as(ry))
+    for n, u, r in zip(("y", "dx", "dalpha", "dbasis"), (y, xx.grad, aa.grad, bb.grad),
+                       (ry, rx.grad, ra.grad, rb.grad)):
+        assert_close(n, u, r, BF)
+
+
+@pytest.mark.parametrize("S,K,act", [(2, 16, "silu"), (3, 7, None), (4, 16, "silu")])
+@pytest.mark.parametrize("B,T,D", [(1, 1, 2), (1, 28, 16), (1, 29, 18), (1, 30, 126), (1, 32, 128),
+                                   (2, 33, 130), (1, 64, 254), (3, 5, 66)])
+def test_stream_edges_fixed(S, K, act, B, T, D):
+    g = gen(100 * S + T)
+    _check(randn(g, B, T, D, scale=0.5), torch.softmax(randn(g, B, T, K), -1),
+           randn(g, K, S, D, scale=0.3), randn(g, B, T, D), act)
+
+
+@pytest.mark.parametrize("S,act", [(2, None), (3, "silu"), (4, "silu"), (4, None)])
+@pytest.mark.parametrize("longest", [3, 45, 700])
+def test_stream_ranges_packed(S, act, longest):
+    # 256 ranges of the two 128-channel groups; two and three steps each
+    g = gen(S * 10 + longest)
+    N, D, K = 256 * 29 * 2 + 77, 130, 12
+    lengths, left = [], N
+    while left:
+        n = min(left, int(torch.randint(1, longest + 1, (1,), generator=g)))
+        lengths.append(n)
+        left -= n
+    _check(randn(g, N, D, scale=0.5), torch.softmax(randn(g, N, K), -1),
+           randn(g, K, S, D, scale=0.3), randn(g, N, D), act, lengths)
+
+
+@pytest.mark.parametrize("form", ["one", "row"])
+def test_stream_broadcast_dy(form):
+    g = gen(7)
+    B, T, D, K, S = 1, 256 * 29 + 1, 258, 16, 4
+    dy = randn(g, 1, 1, 1) if form == "one" else randn(g, 1, 1, D)
+    _check(randn(g, B, T, D, scale=0.5), torch.softmax(randn(g, B, T, K), -1),
+           randn(g, K, S, D, scale=0.3), dy, "silu")
