@@ -370,6 +370,22 @@ int moc_router_backward(const void* z, const void* router, const void* dlogits, 
                         void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * The router of fp32 layers, the same F.linear(z, router) with the activation
+ * after it (moc/api.py:383-388) and its backward on fp32 tensors: out = the
+ * logits (routing 0), softmax_k (1) or exp (2) of them, [n_tokens, k].  Sums are
+ * fp32, drouter's in a fixed order.  k % 4 == 0, k <= 32, z_dim % 64 == 0,
+ * n_tokens * z_dim < 2^29 (moc_router_f32_supported returns 1 for such shapes).
+ * dz or drouter may be NULL.
+ */
+int moc_router_f32_supported(int64_t n_tokens, int64_t z_dim, int64_t k);
+int moc_router_f32_forward(const void* z, const void* router, void* out, int64_t n_tokens,
+                           int64_t z_dim, int64_t k, int routing, void* stream);
+size_t moc_router_f32_backward_workspace_bytes(int64_t n_tokens, int64_t z_dim, int64_t k);
+int moc_router_f32_backward(const void* z, const void* router, const void* dlogits, void* dz,
+                            void* drouter, int64_t n_tokens, int64_t z_dim, int64_t k,
+                            void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Profiling aid; it has no counterpart in the reference.  While set (non-NULL
  * hipEvent_t handles), moc_forward / moc_backward record `start_event` right
  * before and `stop_event` right after their main kernel (the fused forward,

@@ -808,4 +808,49 @@ int moc_router_backward(const void* z, const void* router, const void* dlogits, 
   return hip_status("moc_router_backward launch");
 }
 
+int moc_router_f32_supported(int64_t n_tokens, int64_t z_dim, int64_t k) {
+  return moc::router_f32_supported(n_tokens, z_dim, k) ? 1 : 0;
+}
+
+static int check_router_f32(int64_t n_tokens, int64_t z_dim, int64_t k) {
+  if (moc::router_f32_supported(n_tokens, z_dim, k)) return 0;
+  return fail(MOC_ERR_ARG, "fp32 router shape not supported (n_tokens %lld, z_dim %lld, k %lld): "
+                           "k %% 4 == 0, k <= %d, z_dim %% 64 == 0, n_tokens z_dim < 2^29",
+              (long long)n_tokens, (long long)z_dim, (long long)k, moc::kRouterMaxRoutedK);
+}
+
+int moc_router_f32_forward(const void* z, const void* router, void* out, int64_t n_tokens,
+                           int64_t z_dim, int64_t k, int routing, void* stream) {
+  g_err[0] = '\0';
+  if (const int rc = check_router_f32(n_tokens, z_dim, k)) return rc;
+  if (routing < MOC_ROUTE_ALPHA || routing > MOC_ROUTE_EXP)
+    return fail(MOC_ERR_ARG, "routing must be 0, 1 or 2, got %d", routing);
+  if (!z || !router || !out) return fail(MOC_ERR_ARG, "null tensor pointer");
+  moc::router_f32_forward(z, router, out, n_tokens, z_dim, k, routing, static_cast<hipStream_t>(stream));
+  return hip_status("moc_router_f32_forward launch");
+}
+
+size_t moc_router_f32_backward_workspace_bytes(int64_t n_tokens, int64_t z_dim, int64_t k) {
+  return moc::router_f32_supported(n_tokens, z_dim, k)
+             ? moc::router_f32_backward_workspace(n_tokens, z_dim, k) : 0;
+}
+
+int moc_router_f32_backward(const void* z, const void* router, const void* dlogits, void* dz,
+                            void* drouter, int64_t n_tokens, int64_t z_dim, int64_t k,
+                            void* workspace, size_t workspace_bytes, void* stream) {
+  g_err[0] = '\0';
+  if (const int rc = check_router_f32(n_tokens, z_dim, k)) return rc;
+  if (!router || !dlogits || (drouter && !z)) return fail(MOC_ERR_ARG, "null tensor pointer");
+  if (!dz && !drouter) return 0;
+  if (drouter) {
+    const size_t need = moc::router_f32_backward_workspace(n_tokens, z_dim, k);
+    if (workspace_bytes < need || !workspace)
+      return fail(MOC_ERR_WORKSPACE, "workspace too small: need %zu bytes, got %zu", need,
+                  workspace_bytes);
+  }
+  moc::router_f32_backward(z, router, dlogits, dz, drouter, n_tokens, z_dim, k, workspace,
+                           static_cast<hipStream_t>(stream));
+  return hip_status("moc_router_f32_backward launch");
+}
+
 }  // extern "C"

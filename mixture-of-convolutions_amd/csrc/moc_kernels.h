@@ -176,4 +176,13 @@ void router_forward(const void* z, const void* r, void* out, int64_t N, int64_t 
 void router_backward(const void* z, const void* r, const void* dl, void* dz, void* dr,
                      int64_t N, int64_t Z, int64_t K, void* workspace, hipStream_t st);
 
+// the same for fp32 layers (moc_router_f32.hip): K % 4 == 0, K <= 32, Z % 64 == 0,
+// logits (ROUTE_ALPHA) or weights in fp32; z may be null without dr
+bool router_f32_supported(int64_t N, int64_t Z, int64_t K);
+size_t router_f32_backward_workspace(int64_t N, int64_t Z, int64_t K);
+void router_f32_forward(const void* z, const void* r, void* out, int64_t N, int64_t Z, int64_t K,
+                        int routing, hipStream_t st);
+void router_f32_backward(const void* z, const void* r, const void* dl, void* dz, void* dr,
+                         int64_t N, int64_t Z, int64_t K, void* workspace, hipStream_t st);
+
 }  // namespace moc

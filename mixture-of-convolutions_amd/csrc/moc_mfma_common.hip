@@ -304,18 +304,19 @@ struct Plan {
 };
 
 // The kernels read the caller's weights and basis in place when both already
-// have the operand layout: weights given (no activation to form), bf16
+// have the operand layout: weights given (no activation to form), one dtype
 // everywhere, K = 16 (no padded routes) and 16-byte aligned rows; then no prep
 // launch runs.  The workspace is sized for the prep path either way, since its
 // size is asked for without the pointers.
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
 bool direct(const Problem& p, const void* alpha, const void* basis, const void* dalpha) {
-  // K = 16, 32 or 64: the caller's [N, K] weights and [K, S, D] basis are then the
-  // kernels' padded operand layouts (KP = K) as they are; PATH_MFMA_PREP forces
-  // the prep launch (an A/B switch)
-  return p.path != PATH_MFMA_PREP && route_form(p.routing) == ROUTE_ALPHA && p.x_dt == DT_BF16 &&
-         p.a_dt == DT_BF16 && p.b_dt == DT_BF16 && (p.K == 16 || p.K == 32 || p.K == 64) &&
+  // K = 16, 32 or 64 (fp32: 16 or 32): the caller's [N, K] weights and [K, S, D]
+  // basis are then the kernels' padded operand layouts (KP = K) as they are;
+  // PATH_MFMA_PREP forces the prep launch (an A/B switch)
+  const bool k_ok = p.K == 16 || p.K == 32 || (p.K == 64 && p.x_dt == DT_BF16);
+  return p.path != PATH_MFMA_PREP && route_form(p.routing) == ROUTE_ALPHA &&
+         p.a_dt == p.x_dt && p.b_dt == p.x_dt && k_ok &&
          aligned16(alpha) && aligned16(basis) && aligned16(dalpha);
 }
 
@@ -385,9 +386,10 @@ void launch_stage2(const Problem& p, const Plan& pl, bool dir, char* ws, const v
   const int64_t da_blocks = cdiv(p.n_tokens * 16, 256);
   const int grad = route_grad(p.routing);
   // weights for the activation gradient: prep's fp32 copy, or the caller's
-  // bf16 weights read in place
-  const float* a_r = (grad != ROUTE_ALPHA && !dir)
-                         ? reinterpret_cast<const float*>(ws + pl.off_ar) : nullptr;
+  // weights read in place
+  const float* a_r = grad == ROUTE_ALPHA ? nullptr
+                     : !dir              ? reinterpret_cast<const float*>(ws + pl.off_ar)
+                     : p.x_dt == DT_F32  ? static_cast<const float*>(alpha) : nullptr;
   const auto* a_w = static_cast<const uint16_t*>(alpha);
   const dim3 grid(static_cast<unsigned>(da_blocks + db_blocks));
   const int64_t n_da = pl.bg.gx;

@@ -52,6 +52,8 @@ EXPORTED_SYMBOLS = (
     "moc_router_forward_routed",
     "moc_router_forward_grouped",
     "moc_router_backward_workspace_bytes",
+    "moc_router_f32_supported", "moc_router_f32_forward",
+    "moc_router_f32_backward_workspace_bytes", "moc_router_f32_backward",
     "moc_router_backward",
 )
 
@@ -173,6 +175,14 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.moc_router_backward_workspace_bytes.restype = _z
     lib.moc_router_backward.argtypes = [_p, _p, _p, _p, _p, _l, _l, _l, _i, _p, _z, _p]
     lib.moc_router_backward.restype = _i
+    lib.moc_router_f32_supported.argtypes = [_l, _l, _l]
+    lib.moc_router_f32_supported.restype = _i
+    lib.moc_router_f32_forward.argtypes = [_p, _p, _p, _l, _l, _l, _i, _p]
+    lib.moc_router_f32_forward.restype = _i
+    lib.moc_router_f32_backward_workspace_bytes.argtypes = [_l, _l, _l]
+    lib.moc_router_f32_backward_workspace_bytes.restype = _z
+    lib.moc_router_f32_backward.argtypes = [_p, _p, _p, _p, _p, _l, _l, _l, _p, _z, _p]
+    lib.moc_router_f32_backward.restype = _i
 
 
 def lib() -> ctypes.CDLL:

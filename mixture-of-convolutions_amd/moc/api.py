@@ -8,14 +8,14 @@ the gfx950 HIP kernels of libmoc_hip.so through ``ops`` and
 * the backward recomputes the pre-activation inside the kernel instead of
   re-running the forward (moc/api.py:176-183);
 * the router activation and its gradient cost no kernels of their own
-  (moc/api.py:383-388): for bf16 layers ``MoC.forward`` is one autograd node
-  whose router kernel forms softmax / exp(z . router^T) and whose MoC backward
+  (moc/api.py:383-388): for bf16 and fp32 layers ``MoC.forward`` is one autograd
+  node whose router kernel forms softmax / exp(z . router^T) and whose MoC backward
   returns d(logits) for the router backward; otherwise (and in ``MoC.step``)
   the kernels take the router *logits*, form the weights themselves and
   return d(logits);
 * the router GEMM logits = z . router^T and its backward run on the library's
-  skinny-GEMM kernels for bf16 layers (``router_linear``), torch's F.linear
-  otherwise.
+  skinny-GEMM kernels for bf16 layers (``router_linear``) and inside fp32
+  layers, torch's F.linear otherwise.
 """
 from __future__ import annotations
 
@@ -589,8 +589,9 @@ class MoC(nn.Module):
                                            activation_flag=activation_flag(self.activation),
                                            routing=_ROUTING_CODES[self.router_activation])
                 return y, (cache if output_final_state else None)
-        routed = (self.router.shape[0] <= ops.ROUTER_MAX_ROUTED_K
-                  and ops.router_supported(z, self.router))
+        f32 = ops.router_f32_supported(z, self.router)
+        routed = f32 or (self.router.shape[0] <= ops.ROUTER_MAX_ROUTED_K
+                         and ops.router_supported(z, self.router))
         if cache is None and routed:
             return self._forward_kernels(x, z, output_final_state, cu_seqlens, max_seqlen,
                                          cu_seqlens_cpu, chunk_indices)
@@ -602,7 +603,11 @@ class MoC(nn.Module):
             return _MoCLayerPrefillFunction.apply(x, z, self.router, self.conv_bases, cache,
                                                   self.activation, self.router_activation,
                                                   output_final_state)
-        logits = router_linear(z, self.router)
+        if f32 and cu_seqlens is None and x.dim() == 3 and x.shape[1] == 1:
+            # (a step is not differentiable: no graph to build)
+            logits = ops.router_forward(z.detach(), self.router.detach())
+        else:
+            logits = router_linear(z, self.router)
         return _dispatch(x, logits, self.conv_bases, cache, output_final_state,
                          self.activation, self.router_activation, cu_seqlens, max_seqlen,
                          cu_seqlens_cpu, chunk_indices)

@@ -471,11 +471,36 @@ def _router_shape_supported(z: torch.Tensor, K: int, Z: int) -> bool:
     return hit
 
 
+_router_f32_cache: dict[tuple, bool] = {}
+
+
+def router_f32_supported(z: torch.Tensor, router: torch.Tensor) -> bool:
+    """Whether an fp32 layer's router (GEMM and activation) runs on the library's
+    fp32 router kernels: fp32 z and router on one GPU, k % 4 == 0, k <= 32,
+    z_dim % 64 == 0, no autocast (which has F.linear return 16-bit logits)."""
+    f32 = torch.float32
+    if not z.is_cuda or z.dtype != f32 or router.dtype != f32 or router.device != z.device:
+        return False
+    if torch.is_autocast_enabled("cuda"):
+        return False
+    K, Z = router.shape
+    n = z.numel()
+    if z.shape[-1] != Z or n == 0:
+        return False
+    # the answer depends on the token count through the bound on n_tokens z_dim only
+    key = (Z, K, n < (1 << 29))
+    hit = _router_f32_cache.get(key)
+    if hit is None:
+        hit = bool(_lib.lib().moc_router_f32_supported(n // Z, Z, K))
+        _router_f32_cache[key] = hit
+    return hit
+
+
 def router_forward(z: torch.Tensor, router: torch.Tensor, routing: int = ROUTE_ALPHA
                    ) -> torch.Tensor:
     """logits = z . router^T (the F.linear(z, router) of moc/api.py:383-388);
     with routing 1 / 2 the router activation of moc/api.py:385-388 too:
-    softmax / exp of the bf16 logits, rounded to bf16 (the routing weights)."""
+    softmax / exp of the logits (bf16: of the rounded logits, rounded to bf16)."""
     L = _lib.lib()
     z = z.contiguous()
     r = router.contiguous()
@@ -483,7 +508,10 @@ def router_forward(z: torch.Tensor, router: torch.Tensor, routing: int = ROUTE_A
     N = z.numel() // Z
     out = torch.empty(*z.shape[:-1], K, dtype=z.dtype, device=z.device)
     with _lib.device_guard(z.device):
-        if routing == ROUTE_ALPHA:
+        if z.dtype == torch.float32:
+            rc = L.moc_router_f32_forward(z.data_ptr(), r.data_ptr(), out.data_ptr(), N, Z, K,
+                                          int(routing), _lib.stream_ptr(z.device))
+        elif routing == ROUTE_ALPHA:
             rc = L.moc_router_forward(z.data_ptr(), r.data_ptr(), out.data_ptr(), N, Z, K,
                                       _lib.DT_BF16, _lib.stream_ptr(z.device))
         else:
@@ -556,6 +584,15 @@ def router_backward(z: torch.Tensor, router: torch.Tensor, dlogits: torch.Tensor
     dz = torch.empty_like(z) if need_z else None
     dr = torch.empty_like(r) if need_router else None
     with _lib.device_guard(z.device):
+        if z.dtype == torch.float32:
+            nbytes = L.moc_router_f32_backward_workspace_bytes(N, Z, K) if need_router else 0
+            ws = _workspace(nbytes, z.device)
+            rc = L.moc_router_f32_backward(
+                z.data_ptr(), r.data_ptr(), dl.data_ptr(),
+                None if dz is None else dz.data_ptr(), None if dr is None else dr.data_ptr(),
+                N, Z, K, ws.data_ptr() if nbytes else None, nbytes, _lib.stream_ptr(z.device))
+            _lib.check(rc, "moc_router_f32_backward")
+            return dz, dr
         nbytes = L.moc_router_backward_workspace_bytes(N, Z, K, _lib.DT_BF16) if need_router else 0
         ws = _workspace(nbytes, z.device)
         rc = L.moc_router_backward(
