@@ -1,9 +1,10 @@
-"""Build libmoc_hip.so (gfx950) from csrc/ with hipcc.
+"""Build libmoc_hip.so (gfx950) from csrc/*.hip with hipcc, and the host module
+that calls it, _moc_host.so, from csrc/moc_host.cpp with g++ against torch.
 
     python mixture-of-convolutions_amd/build_lib.py [--jobs N]
 
-Objects go to csrc/_build/, the shared library next to the Python package
-(moc/libmoc_hip.so), where moc/_lib.py loads it.  Every call recompiles.
+Objects go to csrc/_build/, both libraries next to the Python package
+(moc/), where moc/_lib.py loads them.  Every call recompiles.
 """
 from __future__ import annotations
 
@@ -13,12 +14,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_ROOT = Path(__file__).resolve().parent
 CSRC = PKG_ROOT / "csrc"
 BUILD = CSRC / "_build"
 LIB = PKG_ROOT / "moc" / "libmoc_hip.so"
+HOST = PKG_ROOT / "moc" / "_moc_host.so"
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -53,6 +56,34 @@ def _compile(src: Path, extra: tuple[str, ...] = (), build_dir: Path = BUILD) ->
     return obj
 
 
+def _compile_host(build_dir: Path) -> Path:
+    import torch
+    inc = Path(torch.__file__).parent / "include"
+    obj = build_dir / "moc_host.o"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_moc_host",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{inc}", f"-I{inc / 'torch/csrc/api/include'}", f"-I{Path(HIPCC).parents[1] / 'include'}",
+           f"-I{sysconfig.get_path('include')}", "-c", str(CSRC / "moc_host.cpp"), "-o", str(obj)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("moc_host.cpp failed:\n" + res.stdout + res.stderr)
+    return obj
+
+
+def _link_host(obj: Path) -> None:
+    import torch
+    lib = Path(torch.__file__).parent / "lib"
+    tmp = HOST.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-shared", "-o", str(tmp), str(obj), f"-L{lib}", "-ltorch_python",
+           "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", f"-L{LIB.parent}",
+           f"-l:{LIB.name}", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("link of the host module failed:\n" + res.stdout + res.stderr)
+    os.replace(tmp, HOST)
+
+
 def build(jobs: int | None = None, verbose: bool = True, defines: tuple[str, ...] = (),
           out: Path = LIB) -> Path:
     """Compile csrc/*.hip and link ``out``; ``defines`` are extra -D flags."""
@@ -64,7 +95,9 @@ def build(jobs: int | None = None, verbose: bool = True, defines: tuple[str, ...
     jobs = jobs or min(len(sources), max(1, (os.cpu_count() or 4)))
     extra = tuple(f"-D{d}" for d in defines)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_compile_host, build_dir) if Path(out) == LIB else None
         objs = list(ex.map(lambda src: _compile(src, extra, build_dir), sources))
+        host_obj = host.result() if host is not None else None
     LIB_OUT = Path(out)
     tmp = LIB_OUT.with_suffix(".so.tmp")
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
@@ -72,6 +105,8 @@ def build(jobs: int | None = None, verbose: bool = True, defines: tuple[str, ...
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + res.stdout + res.stderr)
     os.replace(tmp, LIB_OUT)
+    if host_obj is not None:
+        _link_host(host_obj)
     if verbose:
         print(f"built {LIB_OUT} from {len(sources)} sources")
     return LIB_OUT

@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib.util
 import threading
 from pathlib import Path
 
@@ -206,6 +207,30 @@ def lib() -> ctypes.CDLL:
                         "`python mixture-of-convolutions_amd/build_lib.py`")
                 _lib = handle
     return _lib
+
+
+HOST_PATH = LIB_PATH.parent / "_moc_host.so"
+_host = None
+
+
+def host():
+    """The host module (csrc/moc_host.cpp) on the loaded library; raises
+    RuntimeError if it is not built."""
+    global _host
+    if _host is None:
+        lib()
+        with _lock:
+            if _host is None:
+                if not HOST_PATH.exists():
+                    raise RuntimeError(
+                        f"{HOST_PATH} is not built; run "
+                        "`python mixture-of-convolutions_amd/build_lib.py` "
+                        "(or __graft_entry__.build()) first")
+                spec = importlib.util.spec_from_file_location("_moc_host", HOST_PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                _host = module
+    return _host
 
 
 @contextlib.contextmanager

@@ -27,7 +27,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd.function import once_differentiable
 
-from . import ops
+from . import _lib, ops
 from ._lib import (ROUTE_ALPHA, ROUTE_EXP, ROUTE_EXP_WEIGHTS, ROUTE_SOFTMAX,
                    ROUTE_SOFTMAX_WEIGHTS)
 from .optim import moc_fan_in_std
@@ -35,6 +35,8 @@ from .optim import moc_fan_in_std
 SUPPORTED_DTYPES = (torch.bfloat16, torch.float32)
 
 _ROUTING_CODES = {"softmax": ROUTE_SOFTMAX, "exp": ROUTE_EXP}
+# activations the host module takes (activation_flag names the others' errors)
+_ACT_CODES = {None: 0, "silu": 1, "swish": 1}
 _WEIGHTS_CODES = {"softmax": ROUTE_SOFTMAX_WEIGHTS, "exp": ROUTE_EXP_WEIGHTS}
 
 
@@ -118,6 +120,19 @@ def _canonicalize_packed_input(x: torch.Tensor, alpha: torch.Tensor
     if x.ndim == 3 and alpha.ndim == 3 and x.shape[0] == 1 and alpha.shape[0] == 1:
         return x[0], alpha[0], True
     raise ValueError("varlen x/alpha must be [N,D]/[N,K] or [1,N,D]/[1,N,K]")
+
+
+def _packed(x, a):
+    """_canonicalize_packed_input, or (None, None, False) where that raises."""
+    if x.ndim == 2 and a.ndim == 2:
+        return x, a, False
+    if x.ndim == 3 and a.ndim == 3 and x.shape[0] == 1 and a.shape[0] == 1:
+        return x[0], a[0], True
+    return None, None, False
+
+
+def _is_length(n) -> bool:
+    return isinstance(n, int) and n > 0
 
 
 def _check_cache(x: torch.Tensor, basis: torch.Tensor, cache: torch.Tensor) -> None:
@@ -537,6 +552,19 @@ def moc_triton(
     """Functional MoC on routing weights (moc/api.py:262-335), backed by the
     HIP kernels.  The name is kept for drop-in compatibility; ``moc_hip`` is the
     same function."""
+    if (x.is_cuda and cache is None and not output_final_state and cu_seqlens_cpu is None
+            and chunk_indices is None and (activation is None or isinstance(activation, str))):
+        # the host module's one call, where the arguments are ones it takes
+        act = _ACT_CODES.get(activation)
+        if act is not None and cu_seqlens is None:
+            y = _lib.host().func(x, alpha, basis, act, None)
+            if y is not None:
+                return y, None
+        elif act is not None and _is_length(max_seqlen):
+            xp, ap, restore = _packed(x, alpha)
+            y = None if xp is None else _lib.host().func(xp, ap, basis, act, cu_seqlens)
+            if y is not None:
+                return (y[None] if restore else y), None
     return _dispatch(x, alpha, basis, cache, output_final_state, activation, None,
                      cu_seqlens, max_seqlen, cu_seqlens_cpu, chunk_indices)
 
@@ -576,6 +604,10 @@ class MoC(nn.Module):
                 max_seqlen: Optional[int] = None, cu_seqlens_cpu: Optional[torch.Tensor] = None,
                 chunk_indices: Optional[torch.Tensor] = None
                 ) -> tuple[torch.Tensor, torch.Tensor | None]:
+        if x.is_cuda and cu_seqlens_cpu is None and chunk_indices is None:
+            out = self._host_forward(x, z, cache, output_final_state, cu_seqlens, max_seqlen)
+            if out is not None:
+                return out
         if cache is not None and cu_seqlens is None:
             # single-token step: router GEMM, router activation and cache update
             # in one launch (the step is not differentiable, as in the reference);
@@ -611,6 +643,30 @@ class MoC(nn.Module):
         return _dispatch(x, logits, self.conv_bases, cache, output_final_state,
                          self.activation, self.router_activation, cu_seqlens, max_seqlen,
                          cu_seqlens_cpu, chunk_indices)
+
+    def _host_forward(self, x, z, cache, want_state, cu_seqlens, max_seqlen):
+        """forward as one call of the host module, or None where the arguments
+        are not ones it takes (the paths below then run, or raise)."""
+        act, code = _ACT_CODES.get(self.activation), _ROUTING_CODES.get(self.router_activation)
+        if act is None or code is None:
+            return None
+        H, router, basis = _lib.host(), self.router, self.conv_bases
+        if cu_seqlens is None:
+            if cache is not None or want_state:
+                out = H.stateful(x, z, router, basis, cache, act, code, want_state)
+                if out is not None or cache is not None:
+                    return out
+            if max_seqlen is not None:
+                return None
+            y = H.layer(x, z, router, basis, act, code, None)
+            if y is None:
+                return None
+            return y, (_final_state(x, None, basis.shape[1]) if want_state else None)
+        if cache is not None or want_state or not _is_length(max_seqlen):
+            return None
+        xp, zp, restore = _packed(x, z)
+        y = None if xp is None else H.layer(xp, zp, router, basis, act, code, cu_seqlens)
+        return None if y is None else ((y[None] if restore else y), None)
 
     def _forward_kernels(self, x, z, output_final_state, cu_seqlens, max_seqlen, cu_seqlens_cpu,
                          chunk_indices):
