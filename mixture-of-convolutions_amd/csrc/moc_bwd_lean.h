@@ -1,12 +1,10 @@
-// Fused backward (stage 1) at four waves per SIMD: bf16 operands, up to 16
-// routes, 2 to 4 taps (the headline layer shape).
+// Fused backward (stage 1) of bf16 layers with 2 to 8 taps and up to 32 routes.
 //
-// What bounds it: instruction issue of four waves per SIMD (a register budget of
-// 128 VGPRs; the two-wave form of bwd_tile, with 32 channels per wave and about
-// 230 VGPRs, issues fp32 work 45% slower).  A wave holds 16 channels, one per
-// lane, and a workgroup of 8 waves the 128 channels of bwd_tile's workgroup, so
-// channel groups, range counts and partial-sum layouts are those of its grid,
-// and stage 2 is the same.
+// What bounds it: instruction issue and the latency chains of two to four waves
+// per SIMD (four, 128 VGPRs, with 2 to 4 taps and 16 routes; else two, 256 VGPRs).
+// A wave holds 16 channels, one per lane, and a workgroup of 8 waves the 128
+// channels of bwd_tile's workgroup, so channel groups, range counts and
+// partial-sum layouts are those of its grids, and stage 2 is the same.
 //
 // A range's rows are cut in four streams of 8 n rows, one per 16-lane group of
 // the wave (lane (j, q): channel j, stream q), walked in n steps of 8 rows.  So
@@ -14,28 +12,37 @@
 // to step: the last S - 1 x rows of the window, and the partial dx of the last
 // S - 1 rows, to which later rows still add (dx[t - off] += g[t] W_{S-1-off}[t]:
 // the same W tile that P uses).  A stream hands what its first rows owe to the
-// rows before them to the stream before it through LDS at the end.  Against
-// super-blocks of 32 consecutive rows (three rows of each recomputed in the next,
-// 11 window rows loaded and converted for 8, a second W tile at shifted rows and
-// a cross-lane read of g for dx) a row takes 25% fewer vector instructions and
-// 8 fewer matrix instructions of 32.  B4 T4096 D2048, 16 routes, 4 taps, both
-// stages: with SiLU 92.3 -> 79.9 us (one-element dy 81.8 -> 73.0), D 4096, 32768
-// tokens, no activation 275.0 -> 262.6 us.
+// rows before them to the stream before it at the end.  Against super-blocks of
+// 32 consecutive rows (S - 1 rows of each recomputed in the next, S + 7 window
+// rows loaded and converted for 8, a second W tile at shifted rows and a
+// cross-lane read of g for dx) a row of 4 taps takes 25% fewer vector
+// instructions and 8 fewer matrix instructions of 32.  And one pass holds every
+// tap and both route chunks, where dx and the m products of more taps or routes
+// ran as two passes with g = dy silu'(P) through memory, or once per route chunk.
+//
+// Both stages, us, before -> here (B4 T4096 D2048, without / with SiLU):
+//   taps       2                3                4                6                8
+//   16 routes  67.5->66.6       77.7->74.7       80.7->75.2       138.7->99.6      151.8->119
+//              72.4->69.7       84.8->77.7       90.6->80.0       157.4->110       201.2->129
+//   32 routes  94.5->82.9       127->94          130->102         161->129         194.6->158
+//              116->85.7        152->95.5        190->109         217->137         252->169
+// and D 4096: 32768 tokens, 16 routes, 4 taps 275 -> 262.6; 16384 tokens, 32
+// routes, 8 taps 335 -> 280.  So it serves every shape it is built for.
 //
 // Work per step and wave (rows 8 i .. 8 i + 7 of each stream):
-//   W_s = alpha . basis_s by MFMA (16x16x16, 16 routes; both operands from LDS,
-//   the basis tile read transposed), P = sum_s W_s x_s, g = dy silu'(P); dx as
-//   above; m_s = g x_s split in bf16 hi / lo; dbasis += alpha^T m_s (16x16x32
-//   over the 32 rows, accumulated over the whole range in registers); dalpha +=
-//   m . basis^T over 16 channels of hi and lo (16x16x32, m read back transposed
-//   from a wave-private LDS tile with ds_read_b64_tr_b16); the 8 waves' dalpha
-//   tiles summed in LDS in wave order.
+//   W_s = alpha . basis_s by MFMA (16x16x16, or 16x16x32 over 32 routes; both
+//   operands from LDS, the basis tile read transposed), P = sum_s W_s x_s, g =
+//   dy silu'(P); dx as above; m_s = g x_s split in bf16 hi / lo; dbasis +=
+//   alpha^T m_s (16x16x32 over the 32 rows, accumulated over the whole range in
+//   registers); dalpha += m . basis^T over 16 channels of hi and lo (16x16x32, m
+//   read back transposed from a wave-private LDS tile with ds_read_b64_tr_b16);
+//   the 8 waves' dalpha tiles summed in LDS in wave order.
 //
-// Measured and not kept: x and dy as one 16-byte load per lane through an LDS
-// tile (4x fewer memory instructions, more LDS work: 81.9 us); the rows' scalar
-// offsets in the accesses' soffset (85.8); the next rows fetched before the m
-// products (no change where it fits the registers, 112 us where it spills); the
-// step loop unrolled twice (no change).
+// Measured and not kept (4 taps, 16 routes, SiLU, 79.9 us): x and dy as one
+// 16-byte load per lane through an LDS tile (4x fewer memory instructions, more
+// LDS work: 81.9); the rows' scalar offsets in the accesses' soffset (85.8); the
+// next rows fetched before the m products (no change where it fits the registers,
+// 112 where it spills); the step loop unrolled twice (no change).
 #pragma once
 
 #include "moc_mfma.h"
@@ -69,14 +76,17 @@ __device__ __forceinline__ f32x4 mma16(s16x4 a, s16x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
-#ifndef MOC_LEAN_WAVES
-#define MOC_LEAN_WAVES 4
-#endif
 constexpr int kLeanWPG = 8;        // waves per workgroup (8 x 16 = 128 channels)
 constexpr int kLeanCW = 16;        // channels per wave
 
-// Shapes the lean pass serves (bf16 operands, single launches).
-constexpr bool bwd_lean(int S, int KC, bool bf) { return bf && KC == 1 && S >= 2 && S <= 4; }
+// Shapes the lean pass serves (bf16 operands).
+constexpr bool bwd_lean(int S, int KC, bool act, bool bf) {
+  return bf && KC <= 2 && S >= 2 && S <= 8;
+}
+// Waves per SIMD it is built for: four (128 VGPRs, two workgroups per CU) with 2
+// to 4 taps and 16 routes, else two (256 VGPRs and up to 156 KB of LDS, one
+// workgroup per CU)
+constexpr int lean_waves(int S, int KC) { return S <= 4 && KC == 1 ? 4 : 2; }
 
 // Rows of a row-major tensor walked with the scalar unit: next(bytes) is a buffer
 // from the current row on (`left` bytes; at most 0 past the end: loads give
@@ -98,7 +108,7 @@ struct RowWalk {
 
 // The work of workgroup (bx, by) of one layer; the __global__ wrappers below
 // map a single launch's 2-D grid or a grouped launch's 1-D grid onto it.
-template <int S, int ACT, bool DY1>
+template <int S, int KC, int ACT, bool DY1>
 __device__ __forceinline__ void
 bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t dys,
               const uint16_t* __restrict__ a_c, const uint16_t* __restrict__ b_c,
@@ -109,21 +119,31 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
   using E = uint16_t;
   using Op = s16x4;
   constexpr int NB = 2, R = 8, TB = 32, H = S - 1, W = R + H;
-  constexpr int KP = 16, WPG = kLeanWPG, CW = kLeanCW;
+  constexpr int KP = 16 * KC, WPG = kLeanWPG, CW = kLeanCW;
   constexpr int ESZ = 2;
-  static_assert(S >= 2 && S <= 4, "lean backward: 2 to 4 taps");
+  static_assert(S >= 2 && S <= 8 && KC <= 2, "lean backward: 2 to 8 taps, up to 32 routes");
+  // the four-wave form leaves what a stream owes its predecessor in LDS
+  constexpr bool kC0Lds = lean_waves(S, KC) == 4;
+  // The next step's rows are loaded where this step's have been converted in the
+  // two-wave form (a SIMD has one other wave to cover the loads: 16 routes, 8
+  // taps 80.9 -> 77.1 us, 32 routes, 4 taps 115.4 -> 109.0), after the m products
+  // in the others (four waves cover them; 8 taps with 32 routes would spill, 167
+  // -> 204 us)
+  constexpr bool kFetchEarly = lean_waves(S, KC) == 2 && !(S == 8 && KC == 2);
 
   // routing-weight rows of a step, unpadded: row rho = 8 q + r is row r of
-  // stream q; the 8-byte chunk c (4 routes) of row rho sits at chunk
-  // c ^ ((rho >> 3) & 3) (W operand, transposed and staging accesses without
-  // bank conflicts)
+  // stream q; the 8-byte chunk c (4 routes) of row rho sits at chunk c ^ asw(rho)
+  // (W operand, transposed and staging accesses without bank conflicts)
+  auto asw = [](int row) -> int {
+    return KC == 1 ? (row >> 3) & 3 : ((row >> 1) & 1) | (((row >> 3) & 3) << 1);
+  };
   __shared__ __align__(16) E a_lds[2][TB][KP];
   __shared__ __align__(16) Op m_tr[WPG][2][TrTile1::kSlots];  // [wave][hi / lo]
-  // dalpha B operands of each wave, b_lds[wave][s][k = j][4 channels, chunk
-  // q ^ (j / 4)] (a 16-lane group of a read touches 16 distinct slots)
-  __shared__ __align__(16) Op b_lds[WPG][S][16 * 4];
-  __shared__ float da_lds[2][WPG][NB][16][17];
-  __shared__ float c0_lds[H][64 * WPG];
+  // basis tile of each wave, b_lds[wave][s][kc][route j][4 channels, chunk q ^
+  // (j / 4)] (a 16-lane group of a read touches 16 distinct slots)
+  __shared__ __align__(16) Op b_lds[WPG][S][KC][16 * 4];
+  __shared__ float da_lds[2][WPG][NB][KC][16][17];
+  __shared__ float c0_lds[kC0Lds ? H : 1][kC0Lds ? 64 * WPG : 1];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -180,19 +200,23 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
     const int64_t ch = d0 + 4 * q;
     const bool on = wave_on && ch < D;
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      Op bda;
-      bb.load<8>(row_off(j * S + s, 0, rb, static_cast<uint32_t>(ch * ESZ), on), &bda);
-      if (ch + 2 >= D) {
-        bda[2] = 0;
-        bda[3] = 0;
-      }
-      b_lds[wave][s][j * 4 + (q ^ (j >> 2))] = bda;
-    }
-  }
-  f32x4 dbacc[S];
+    for (int s = 0; s < S; ++s)
 #pragma unroll
-  for (int s = 0; s < S; ++s) dbacc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int kc = 0; kc < KC; ++kc) {
+        Op bda;
+        bb.load<8>(row_off((16 * kc + j) * S + s, 0, rb, static_cast<uint32_t>(ch * ESZ), on), &bda);
+        if (ch + 2 >= D) {
+          bda[2] = 0;
+          bda[3] = 0;
+        }
+        b_lds[wave][s][kc][j * 4 + (q ^ (j >> 2))] = bda;
+      }
+  }
+  f32x4 dbacc[S][KC];
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) dbacc[s][kc] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // raw rows of one step
   E xr[R], dr[DY1 ? 1 : R];
@@ -213,8 +237,8 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
       }
     }
   };
-  // routing-weight rows of a step: 32 x 16 elements, 8 bytes per thread of the
-  // first two waves (row rho: thread rho 4 + chunk)
+  // routing-weight rows of a step: 32 rows, 8 bytes per thread of the first 2 KC
+  // waves (row rho: thread 4 KC rho + chunk)
   // (the per-lane terms are formed where they are used, from an opaque copy of
   // the thread id: hoisted out of the loop they outgrow the register budget)
   auto opaque_tid = [&]() {
@@ -222,20 +246,20 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
     asm volatile("" : "+v"(t));
     return t;
   };
-  static_assert(TB * KP / 4 == 128, "two waves fetch a step's routing weights");
+  static_assert(TB * KP / 4 == 128 * KC, "2 KC waves fetch a step's routing weights");
   RowWalk aw{reinterpret_cast<const char*>(a_c + first * KP), static_cast<int32_t>((row_hi - first) * KP * ESZ)};
   E arw[4];
   auto fetch_a = [&]() {
     const Buf ab = aw.next(R * KP * ESZ);
-    if (wave < 2) {
-      const int t = opaque_tid(), row = t >> 2;
-      ab.load<8>(static_cast<uint32_t>((R * n * (row >> 3) + (row & 7)) * KP * ESZ + (t & 3) * 8), arw);
+    if (wave < 2 * KC) {
+      const int t = opaque_tid(), row = t / (4 * KC);
+      ab.load<8>(static_cast<uint32_t>((R * n * (row >> 3) + (row & 7)) * KP * ESZ + (t % (4 * KC)) * 8), arw);
     }
   };
   auto stage_alpha = [&](int buf) {
-    if (wave < 2) {
-      const int t = opaque_tid(), row = t >> 2;
-      Vec<E, 4>::store(&a_lds[buf][row][((t & 3) ^ ((row >> 3) & 3)) * 4], arw);
+    if (wave < 2 * KC) {
+      const int t = opaque_tid(), row = t / (4 * KC);
+      Vec<E, 4>::store(&a_lds[buf][row][((t % (4 * KC)) ^ asw(row)) * 4], arw);
     }
   };
 
@@ -264,13 +288,13 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
   int32_t ns = start_from(srow - (S - 2));
 
   // dx rows -(S-1) .. R-1 of a step: dxa[w] is row w - (S-1); the first S-1 carry
-  // over from the step before.  c0_lds: what a stream's first rows add to the
-  // rows before it, which the stream before takes at the end
-  float dxa[W];
+  // over from the step before.  c0 / c0_lds: what a stream's first rows add to
+  // the rows before it, which the stream before takes at the end
+  float dxa[W], c0[H];
 #pragma unroll
-  for (int e = 0; e < H; ++e) dxa[R + e] = 0.f;
+  for (int e = 0; e < H; ++e) dxa[R + e] = c0[e] = 0.f;
 
-  // dalpha partials of this channel group from row `first` on (own rows, 16 routes)
+  // dalpha partials of this channel group from row `first` on (own rows)
   RowWalk pdw{reinterpret_cast<const char*>(part_da + (static_cast<int64_t>(bx) * N + first) * KP),
               static_cast<int32_t>((own_hi - first) * KP * 4)};
 
@@ -293,16 +317,27 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
     }
     // (unconditionally, also after the last step: rows past the buffer load zeros)
     fetch_a();
+    if constexpr (kFetchEarly) {
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_xdy();
+      __builtin_amdgcn_sched_barrier(0);
+    }
 
-    // alpha operand of token block b: row 8 (j / 4) + 4 b + j % 4, chunk q ^ (j / 4)
-    Op aop[NB];
+    // alpha operand of token block b: row 8 (j / 4) + 4 b + j % 4, chunk 4 kc + q
+    Op aop[NB][KC];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
-      aop[b] = *reinterpret_cast<const Op*>(&a_lds[buf][R * (j >> 2) + 4 * b + (j & 3)][(q ^ (j >> 2)) * 4]);
-
-    f32x4 dacc[NB];
 #pragma unroll
-    for (int b = 0; b < NB; ++b) dacc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int kc = 0; kc < KC; ++kc) {
+        const int row = R * (j >> 2) + 4 * b + (j & 3);
+        aop[b][kc] = *reinterpret_cast<const Op*>(&a_lds[buf][row][((4 * kc + q) ^ asw(row)) * 4]);
+      }
+
+    f32x4 dacc[NB][KC];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) dacc[b][kc] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     {
       // bit k of `sbm`: window row t0 - (S-1) + k starts a segment; bit r of
@@ -332,17 +367,27 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
         }
       };
 
-      // basis[4 q + v, s, channel j]: the tile's rows read transposed
-      Op bop[S];
+      // W of tap s for this lane's rows; the basis operand (routes 16 kc + 4 q + v,
+      // channel j) is the tile's rows read transposed.  With the activation P and
+      // dx read the same W tiles; without, over 32 routes, dx forms each where it
+      // reads it
+      auto form_w = [&](int s, f32x4 (&w)[NB]) {
+        Op bop[KC];
 #pragma unroll
-      for (int s = 0; s < S; ++s)
-        bop[s] = TrTile<NB, 2>::read(&b_lds[wave][s][(4 * q + (j >> 2)) * 4 + ((j & 3) ^ q)]);
-      // W of this lane's rows: P and dx both read it
-      f32x4 w4[S][NB];
+        for (int kc = 0; kc < KC; ++kc)
+          bop[kc] = TrTile<NB, 2>::read(&b_lds[wave][s][kc][(4 * q + (j >> 2)) * 4 + ((j & 3) ^ q)]);
 #pragma unroll
-      for (int s = 0; s < S; ++s)
+        for (int b = 0; b < NB; ++b) {
+          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (KC == 2) w[b] = mma32(aop[b][0], aop[b][1], bop[0], bop[1], zero);
+          else w[b] = mma16(aop[b][0], bop[0], zero);
+        }
+      };
+      constexpr bool kKeepW = ACT != 0 || KC == 1;
+      f32x4 w4[kKeepW ? S : 1][NB];
+      if constexpr (kKeepW)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) w4[s][b] = mma16(aop[b], bop[s], f32x4{0.f, 0.f, 0.f, 0.f});
+        for (int s = 0; s < S; ++s) form_w(s, w4[s]);
 
       if constexpr (ACT != 0) if (act) {  // (act: uniform; always with a fixed ACT)
         float p[R];
@@ -352,7 +397,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
         for (int s = 0; s < S; ++s)
 #pragma unroll
           for (int r = 0; r < R; ++r)
-            if (tap_ok(r, s)) p[r] = fmaf(xw[r + s], w4[s][r >> 2][r & 3], p[r]);
+            if (tap_ok(r, s)) p[r] = fmaf(xw[r + s], w4[kKeepW ? s : 0][r >> 2][r & 3], p[r]);
         // g *= silu'(P) = sg (1 + P (1 - sg)), sg = sigmoid(P) as sigmoid_f forms it
         float sg[R];
 #pragma unroll
@@ -371,14 +416,20 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
 #pragma unroll
         for (int r = 0; r < R; ++r) dxa[H + r] = 0.f;
 #pragma unroll
-        for (int off = 0; off < S; ++off)
+        for (int off = 0; off < S; ++off) {
+          const int s = S - 1 - off;
+          if constexpr (!kKeepW) form_w(s, w4[0]);
 #pragma unroll
           for (int r = 0; r < R; ++r)
-            if (tap_ok(r, S - 1 - off))
-              dxa[H + r - off] = fmaf(g[r], w4[S - 1 - off][r >> 2][r & 3], dxa[H + r - off]);
+            if (tap_ok(r, s))
+              dxa[H + r - off] = fmaf(g[r], w4[kKeepW ? s : 0][r >> 2][r & 3], dxa[H + r - off]);
+        }
         if (i == 0) {
 #pragma unroll
-          for (int e = 0; e < H; ++e) c0_lds[e][tl] = dxa[e];
+          for (int e = 0; e < H; ++e) {
+            if constexpr (kC0Lds) c0_lds[e][tl] = dxa[e];
+            else c0[e] = dxa[e];
+          }
         }
         // rows -(S-1) .. R-S of the step are complete; before the first step's
         // they belong to the stream (or range) before
@@ -392,15 +443,24 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
       // alpha^T operands of the dbasis MFMA, own rows only (the last step's
       // final S-1 rows of stream 3 are the next range's; rows past N are zero):
       // at[b] = alpha[row 8 q + 4 b + v, j] (transposed read of the staged rows)
-      Op at[NB];
+      Op at[NB][KC];
 #pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const int r = R * q + 4 * b + (j >> 2);
-        at[b] = TrTile<NB, 2>::read(&a_lds[buf][r][((j & 3) ^ q) * 4]);
-      }
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) {
+          const int row = R * q + 4 * b + (j >> 2);
+          at[b][kc] = TrTile<NB, 2>::read(&a_lds[buf][row][((4 * kc + (j & 3)) ^ asw(row)) * 4]);
+        }
       if (!more) {
-        const uint64_t keep = q == 3 ? ((1ull << (16 * (4 - H))) - 1ull) : ~0ull;
-        at[NB - 1] = __builtin_bit_cast(Op, __builtin_bit_cast(uint64_t, at[NB - 1]) & keep);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          constexpr int kOwn = R - H;  // rows of stream 3 that are still this range's
+          const int n_ok = kOwn - 4 * b < 0 ? 0 : (kOwn - 4 * b < 4 ? kOwn - 4 * b : 4);
+          const uint64_t keep = q == 3 && n_ok < 4 ? ((1ull << (16 * n_ok)) - 1ull) : ~0ull;
+#pragma unroll
+          for (int kc = 0; kc < KC; ++kc)
+            at[b][kc] = __builtin_bit_cast(Op, __builtin_bit_cast(uint64_t, at[b][kc]) & keep);
+        }
       }
       // m of tap s -> hi / lo operands -> this wave's tile, dbasis MFMAs
       auto stage_m = [&](int s) {
@@ -421,15 +481,18 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
           m_tr[wave][0][TrTile1::wslot(j, q, b)] = mh[b];
           m_tr[wave][1][TrTile1::wslot(j, q, b)] = ml[b];
         }
-        dbacc[s] = mma32(mh[0], mh[1], at[0], at[1], dbacc[s]);
-        dbacc[s] = mma32(ml[0], ml[1], at[0], at[1], dbacc[s]);
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) {
+          dbacc[s][kc] = mma32(mh[0], mh[1], at[0][kc], at[1][kc], dbacc[s][kc]);
+          dbacc[s][kc] = mma32(ml[0], ml[1], at[0][kc], at[1][kc], dbacc[s][kc]);
+        }
       };
       // dalpha contracts 16 channels of the hi and of the lo part in one
       // 16x16x32 MFMA against the basis operand twice.  The transposed reads of
       // a tap (ra[rb][h] = m[16 rb + i][4 qq + {0..3}]) are issued before the next
       // tap's m values are formed and written (a wave's LDS operations complete
       // in issue order, so one tile serves)
-      Op ra[NB][2], bda;
+      Op ra[NB][2], bda[KC];
       stage_m(0);
 #pragma unroll
       for (int s = 0; s < S; ++s) {
@@ -439,37 +502,47 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
 #pragma unroll
           for (int h = 0; h < 2; ++h)
             ra[r2][h] = TrTile<NB, 2>::read(&m_tr[wave][h][TrTile1::rslot(j, q, r2)]);
-        bda = b_lds[wave][s][j * 4 + (q ^ (j >> 2))];
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) bda[kc] = b_lds[wave][s][kc][j * 4 + (q ^ (j >> 2))];
         __builtin_amdgcn_sched_barrier(0);
         if (s + 1 < S) stage_m(s + 1);
 #pragma unroll
-        for (int r2 = 0; r2 < NB; ++r2) dacc[r2] = mma32(ra[r2][0], ra[r2][1], bda, bda, dacc[r2]);
+        for (int r2 = 0; r2 < NB; ++r2)
+#pragma unroll
+          for (int kc = 0; kc < KC; ++kc)
+            dacc[r2][kc] = mma32(ra[r2][0], ra[r2][1], bda[kc], bda[kc], dacc[r2][kc]);
       }
       wave_lds_sync();
     }
-    // the next step's rows, into the registers the raw rows left
-    // (unconditionally, as fetch_a above); issued after the m products, where
-    // the fewest registers are live, and covered by the other waves of the SIMD
-    fetch_xdy();
+    // (unconditionally, as fetch_a above); after the m products, where the fewest
+    // registers are live
+    if constexpr (!kFetchEarly) fetch_xdy();
 
 #pragma unroll
     for (int r2 = 0; r2 < NB; ++r2)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) da_lds[buf][wave][r2][4 * q + v][j] = dacc[r2][v];
+      for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) da_lds[buf][wave][r2][kc][4 * q + v][j] = dacc[r2][kc][v];
     if (more) stage_alpha(buf ^ 1);
     __syncthreads();
     // sum the 8 waves' dalpha tiles in wave order; rows past the own ones drop
     {
-      const int r2 = tl >> 8, row = (tl >> 4) & 15, c = tl & 15;
-      float tv[WPG];
+      const int r2 = tl >> 8, row = (tl >> 4) & 15, c = tl & 15, rho = tl >> 4;
+      const Buf pdb = pdw.next(R * KP * 4);
+      const uint32_t off = static_cast<uint32_t>(((R * n * (rho >> 3) + (rho & 7)) * KP + c) * 4);
+      float tv[KC][WPG];
 #pragma unroll
-      for (int w = 0; w < WPG; ++w) tv[w] = da_lds[buf][w][r2][row][c];
-      float sum = 0.f;
+      for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
-      for (int w = 0; w < WPG; ++w) sum += tv[w];
-      const int rho = tl >> 4;
-      pdw.next(R * KP * 4)
-          .store<4>(static_cast<uint32_t>(((R * n * (rho >> 3) + (rho & 7)) * KP + c) * 4), &sum);
+        for (int w = 0; w < WPG; ++w) tv[kc][w] = da_lds[buf][w][r2][kc][row][c];
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < WPG; ++w) sum += tv[kc][w];
+        pdb.store<4>(off + 64 * kc, &sum);
+      }
     }
   };
   // plain steps in a loop of their own: the accumulators stay in their registers
@@ -485,35 +558,41 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
   if (dxv != nullptr) {
 #pragma unroll
     for (int e = 0; e < H; ++e) {
-      const E o = f32_to_bf16(dxa[R + e] + c0_lds[e][(tid & ~63) | ((lane + 16) & 63)]);
+      const int from = (lane + 16) & 63;
+      const float owed = kC0Lds ? c0_lds[kC0Lds ? e : 0][kC0Lds ? (tid & ~63) | from : 0] : __shfl(c0[e], from, 64);
+      const E o = f32_to_bf16(dxa[R + e] + owed);
       dxw.next(rb).store<ESZ>(vx, &o);
     }
   }
 
-  // this workgroup's dbasis partial: dbacc[s][v] is (k = j, s, channel d0 + 4 q + v);
-  // with D % 4 == 2 the rows are 8-byte aligned and the last group of 4 half past D
+  // this workgroup's dbasis partial: dbacc[s][kc][v] is (k = 16 kc + j, s, channel
+  // d0 + 4 q + v); with D % 4 == 2 the rows are 8-byte aligned and the last group
+  // of 4 half past D
   if (wave_on && d0 + 4 * q < D) {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      float* dst = part_db + ((static_cast<int64_t>(by) * KP + j) * S + s) * D + d0 + 4 * q;
-      if (D % 4 == 0) {
-        *reinterpret_cast<f32x4*>(dst) = dbacc[s];
-      } else {
-        *reinterpret_cast<f32x2*>(dst) = f32x2{dbacc[s][0], dbacc[s][1]};
-        if (d0 + 4 * q + 2 < D) *reinterpret_cast<f32x2*>(dst + 2) = f32x2{dbacc[s][2], dbacc[s][3]};
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) {
+        const f32x4 v = dbacc[s][kc];
+        float* dst = part_db + ((static_cast<int64_t>(by) * KP + 16 * kc + j) * S + s) * D + d0 + 4 * q;
+        if (D % 4 == 0) {
+          *reinterpret_cast<f32x4*>(dst) = v;
+        } else {
+          *reinterpret_cast<f32x2*>(dst) = f32x2{v[0], v[1]};
+          if (d0 + 4 * q + 2 < D) *reinterpret_cast<f32x2*>(dst + 2) = f32x2{v[2], v[3]};
+        }
       }
-    }
   }
 }
 
-template <int S, bool ACT, bool DY1>
-__global__ void __launch_bounds__(64 * kLeanWPG) __attribute__((amdgpu_waves_per_eu(MOC_LEAN_WAVES)))
+template <int S, int KC, bool ACT, bool DY1>
+__global__ void __launch_bounds__(64 * kLeanWPG) __attribute__((amdgpu_waves_per_eu(lean_waves(S, KC))))
 bwd_lean_kernel(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t dys,
                 const uint16_t* __restrict__ a_c, const uint16_t* __restrict__ b_c,
                 void* __restrict__ dxv, float* __restrict__ part_da, float* __restrict__ part_db,
                 SeqLayout seq, int64_t D, int gy, int gy1, int n_old, int n_total) {
-  bwd_lean_tile<S, ACT, DY1>(xv, dyv, dys, a_c, b_c, dxv, part_da, part_db, seq, D,
+  bwd_lean_tile<S, KC, ACT, DY1>(xv, dyv, dys, a_c, b_c, dxv, part_da, part_db, seq, D,
                         static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), gy, gy1, n_old,
                         n_total);
 }
@@ -521,8 +600,8 @@ bwd_lean_kernel(const void* __restrict__ xv, const void* __restrict__ dyv, int64
 // Several layers in one launch (1-D grid, the layers' grids one after another,
 // as bwd_layers_kernel maps them), so that a grouped launch returns the
 // per-layer calls' results bit for bit.
-template <int S, int ACT, bool DY1>
-__global__ void __launch_bounds__(64 * kLeanWPG) __attribute__((amdgpu_waves_per_eu(MOC_LEAN_WAVES)))
+template <int S, int KC, int ACT, bool DY1>
+__global__ void __launch_bounds__(64 * kLeanWPG) __attribute__((amdgpu_waves_per_eu(lean_waves(S, KC))))
 bwd_lean_layers_kernel(BwdLayers ly, SeqLayout seq) {
   const int blk = static_cast<int>(blockIdx.x);
   const BwdLayer* Lp = &ly.l[layer_index(ly, blk)];
@@ -532,7 +611,7 @@ bwd_lean_layers_kernel(BwdLayers ly, SeqLayout seq) {
     local -= gxl;
     ++row;
   }
-  bwd_lean_tile<S, ACT, DY1>(Lp->x, Lp->dy, Lp->dys, static_cast<const uint16_t*>(Lp->a),
+  bwd_lean_tile<S, KC, ACT, DY1>(Lp->x, Lp->dy, Lp->dys, static_cast<const uint16_t*>(Lp->a),
                         static_cast<const uint16_t*>(Lp->b), Lp->dx, Lp->part_da, Lp->part_db, seq,
                         Lp->D, local, row, Lp->gy, Lp->gy1, Lp->n_old, Lp->n_total, Lp->act != 0);
 }

@@ -755,12 +755,15 @@ bool layers_grouped(const Problem* ps, int n, bool backward) {
 
 namespace {
 // Stage-1 class of a layer in a grouped backward: its route chunks, and its
-// activation where either activation's layers run a two-pass form (the two
-// forms, or a two-pass and a fused one, cannot share a launch).
+// activation where either activation's layers run a two-pass form, or only one
+// of them the lean pass (different forms cannot share a launch).
 int bwd_class(const Problem& p) {
   const int S = static_cast<int>(p.S), KC = route_chunks(p.K);
-  const bool two = bwd_two_pass(S, KC, false, true) || bwd_two_pass_r(S, KC, false, true) ||
-                   bwd_two_pass_g(S, KC, true, true);
+  const bool lean0 = bwd_lean(S, KC, false, true);
+  const bool lean1 = bwd_lean(S, KC, true, true);
+  const bool two = lean0 != lean1 ||
+                   (!lean0 && (bwd_two_pass(S, KC, false, true) || bwd_two_pass_r(S, KC, false, true) ||
+                               bwd_two_pass_g(S, KC, true, true)));
   const int act = two ? (p.activation != 0 ? 1 : 0) : 2;
   return KC * 4 + act;
 }

@@ -31,10 +31,6 @@ constexpr int fwd_nb(int S) { return S == 8 ? MOC_FWD_NB8 : kFwdNB; }
 constexpr int kBwdNB = 2, kBwdNC = 2, kBwdWPG = MOC_BWD_WPG;
 static_assert(kLeanWPG * kLeanCW == 16 * kBwdNC * MOC_BWD_WPG,
               "the lean backward covers the channel groups of the fused pass's grid");
-// the lean fused backward (moc_bwd_lean.h) for the shapes it serves; 0: bwd_tile's
-#ifndef MOC_BWD_LEAN
-#define MOC_BWD_LEAN 1
-#endif
 // Resident workgroups the grids are sized for (256 CUs).
 #ifndef MOC_FWD_TARGET_WG
 #define MOC_FWD_TARGET_WG 2048
@@ -178,31 +174,12 @@ inline Grid2 bwd_grid_tiered(int64_t N, int64_t gx, int64_t D, int64_t S, int n_
   return g;
 }
 
-// Grid of the lean fused pass (moc_bwd_lean.h): the channel groups, range count
-// and tiers above, but counted in steps of 32 rows of which a range gives up
-// S - 1 in all (n steps own 32 n - (S - 1) rows; range by starts at row
-// 32 steps_before - by (S - 1)).  Every range has at least one step: there are
-// at most ceil(N / (32 - (S - 1))) ranges.
-inline Grid2 bwd_lean_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int n_cu) {
-  Grid2 g = bwd_grid_tiered(N, gx, D, S, n_cu);
-  const int64_t gy = g.gy, gy1 = g.gy1;
-  const int64_t steps = cdiv(N + gy * (S - 1), 16 * kBwdNB);
-  const int64_t n_old = (steps * kBwdOldShare + 50) / 100;
-  if (gy1 < gy && n_old >= gy1 && steps - n_old >= gy - gy1) {
-    g.n_old = static_cast<int>(n_old);
-  } else {
-    g.gy1 = static_cast<int>(gy);
-    g.n_old = static_cast<int>(steps);
-  }
-  g.n_total = static_cast<int>(steps);
-  return g;
-}
-
 // The backward in two passes (bwd_kernel modes kBwdDx, then kBwdTaps with the
-// taps split in halves) where the fused pass does not fit two waves per SIMD
-// and no activation needs P: bf16, 32 routes and 4 to 8 taps, 16 routes and 7
-// or 8 taps (measured against the fused pass at every kernel size: below those
-// the fused pass is faster).
+// taps split in halves) where the lean pass is not built, the fused pass of
+// bwd_tile does not fit two waves per SIMD and no activation needs P: bf16, the
+// prefill with 32 routes and 4 to 8 taps or 16 routes and 7 or 8 taps (measured
+// against the fused pass at every kernel size: below those the fused pass is
+// faster), and 9 to 16 taps.
 // fp32 (the same two passes on fp32 operands, with and without the activation):
 // 16 routes from 5 taps (4 without the activation) to 16, 32 routes from 4 to
 // 8 taps.  Past 8 taps the fused fp32 tile does not build (its register file);
@@ -218,8 +195,8 @@ constexpr bool bwd_two_pass(int S, int KC, bool act, bool bf) {
   return !act && ((bf && ((KC == 2 && S >= 4) || (KC == 1 && S >= 7))) || (!bf && f32_two_pass(S, KC, act)));
 }
 // With the activation, the two passes where the fused pass spills or forms the
-// same work per route chunk (bf16: 32 routes and 5 to 8 taps, 16 routes and 8,
-// 64 routes and 3 to 8; measured against the fused pass at each size): the dx
+// same work per route chunk (bf16: 64 routes and 3 to 8 taps, 9 to 16 taps, and
+// of the prefill's shapes below 32 routes; measured against the fused pass): the dx
 // pass forms g = dy silu'(P) and leaves it in the workspace (fp32 [N, D]) for the
 // taps pass.  Single launches only (the grouped launch keeps the fused pass).
 constexpr bool bwd_two_pass_g(int S, int KC, bool act, bool bf) {
@@ -233,9 +210,13 @@ constexpr bool bwd_two_pass_g(int S, int KC, bool act, bool bf) {
 // 257 / 335 / 429).
 constexpr bool pre_two_pass_g(int S, int KC) { return (KC == 2 && S >= 6) || KC == 4; }
 // (the prefill passes are built for bf16: fp32 prefill keeps the fused pass)
+inline bool bwd_lean(const Problem& p) {
+  return !p.pre &&
+         bwd_lean(static_cast<int>(p.S), route_chunks(p.K), p.activation != 0, p.x_dt == DT_BF16);
+}
 inline bool bwd_two_pass_g(const Problem& p) {
   const int S = static_cast<int>(p.S), KC = route_chunks(p.K);
-  return (!p.pre || (pre_two_pass_g(S, KC) && p.x_dt == DT_BF16)) &&
+  return !bwd_lean(p) && (!p.pre || (pre_two_pass_g(S, KC) && p.x_dt == DT_BF16)) &&
          bwd_two_pass_g(S, KC, p.activation != 0, p.x_dt == DT_BF16);
 }
 // 64 routes without activation: the two passes, the taps pass split in route
@@ -247,8 +228,8 @@ constexpr bool pre_two_pass_r(int S) { return S >= 2; }
 inline bool bwd_two_pass(const Problem& p) {
   const int S = static_cast<int>(p.S), KC = route_chunks(p.K);
   const bool act = p.activation != 0, bf = p.x_dt == DT_BF16;
-  return (bwd_two_pass(S, KC, act, bf) && (bf || !p.pre)) || bwd_two_pass_g(p) ||
-         ((!p.pre || pre_two_pass_r(S)) && bwd_two_pass_r(S, KC, act, bf));
+  return !bwd_lean(p) && ((bwd_two_pass(S, KC, act, bf) && (bf || !p.pre)) || bwd_two_pass_g(p) ||
+                          ((!p.pre || pre_two_pass_r(S)) && bwd_two_pass_r(S, KC, act, bf)));
 }
 // route parts of the taps pass's grid (halves with 64 routes), whose single
 // round of workgroups then covers half as many tiles
@@ -262,9 +243,34 @@ inline Grid2 bwd_taps_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int n_cu
   return bwd_grid_gx(N, gx, D, S, n_cu > 0 ? int64_t(n_cu) * kTapsPerCU : kBwdTargetWG / 2, true);
 }
 
+// Grid of the lean fused pass (moc_bwd_lean.h): channel groups, range counts and
+// tiers of the grids above (two workgroups per CU for its four-wave form, one for
+// the two-wave form), but counted in steps of 32 rows of which a range gives up
+// S - 1 in all (n steps own 32 n - (S - 1) rows; range by starts at row
+// 32 steps_before - by (S - 1)).  Every range has at least one step: there are
+// at most ceil(N / (32 - (S - 1))) ranges.
+inline Grid2 bwd_lean_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int KC, int n_cu) {
+  const bool four = lean_waves(static_cast<int>(S), KC) == 4;
+  Grid2 g = four ? bwd_grid_tiered(N, gx, D, S, n_cu) : bwd_taps_grid(N, gx, D, S, n_cu);
+  const int64_t gy = g.gy, gy1 = g.gy1;
+  const int64_t steps = cdiv(N + gy * (S - 1), 16 * kBwdNB);
+  const int64_t n_old = (steps * kBwdOldShare + 50) / 100;
+  if (gy1 < gy && n_old >= gy1 && steps - n_old >= gy - gy1) {
+    g.n_old = static_cast<int>(n_old);
+  } else {
+    g.gy1 = static_cast<int>(gy);
+    g.n_old = static_cast<int>(steps);
+  }
+  g.n_total = static_cast<int>(steps);
+  return g;
+}
+
 // The grid whose workgroups own the dalpha / dbasis partials (workspace,
-// stage 2): the taps pass's for the two-pass form, else the fused pass's.
+// stage 2): the lean pass's, the taps pass's for the two-pass form, else the
+// fused pass's.
 inline Grid2 bwd_partials_grid(const Problem& p) {
+  if (bwd_lean(p))
+    return bwd_lean_grid(p.n_tokens, cdiv(p.D, kBwdCW), p.D, p.S, route_chunks(p.K), device_cu_count());
   return bwd_two_pass(p) ? bwd_taps_grid(p.n_tokens, cdiv(p.D, kTapsCW), p.D, p.S,
                                          device_cu_count() / taps_route_parts(route_chunks(p.K)))
                          : bwd_grid_gx(p.n_tokens, cdiv(p.D, kBwdCW), p.D, p.S);
@@ -311,14 +317,14 @@ void bwd_one(const Problem& p, const void* x, const void* dy, const void* a_c, c
   else {
   using E = typename CT<BF>::elem;
   constexpr bool kSplit = BF && KC >= 2;
-  constexpr bool kTwo = bwd_two_pass(S, KC, ACT, BF) || bwd_two_pass_g(S, KC, ACT, BF) ||
-                        bwd_two_pass_r(S, KC, ACT, BF);
-  // the fused pass at four waves per SIMD (moc_bwd_lean.h) where it is built
-  constexpr bool kLean = MOC_BWD_LEAN && !kTwo && bwd_lean(S, KC, BF);
+  // the fused pass in streams (moc_bwd_lean.h) where it is the faster one
+  constexpr bool kLean = bwd_lean(S, KC, ACT, BF);
+  constexpr bool kTwo = !kLean && (bwd_two_pass(S, KC, ACT, BF) || bwd_two_pass_g(S, KC, ACT, BF) ||
+                                   bwd_two_pass_r(S, KC, ACT, BF));
   // tiers for the fused pass at two resident workgroups per CU (not split in route chunks)
   constexpr bool kTiers = !kTwo && !kSplit && kBwdMinWaves<S, KC, kBwdFused, BF> == 2;
   const int64_t gx_all = cdiv(p.D, kBwdCW);
-  const Grid2 g = kLean    ? bwd_lean_grid(p.n_tokens, gx_all, p.D, S, device_cu_count())
+  const Grid2 g = kLean    ? bwd_lean_grid(p.n_tokens, gx_all, p.D, S, KC, device_cu_count())
                   : kTiers ? bwd_grid_tiered(p.n_tokens, gx_all, p.D, S, device_cu_count())
                            : bwd_grid(p.n_tokens, p.D, S);
   const auto* a = static_cast<const E*>(a_c);
@@ -349,7 +355,7 @@ void bwd_one(const Problem& p, const void* x, const void* dy, const void* a_c, c
   } else if constexpr (kLean) {
     // (the lean pass's workgroup covers the same kBwdCW channels with 8 waves)
     // (one dy element for every token and channel: its own instantiation)
-    auto kern = p.dy_stride < 0 ? bwd_lean_kernel<S, ACT, true> : bwd_lean_kernel<S, ACT, false>;
+    auto kern = p.dy_stride < 0 ? bwd_lean_kernel<S, KC, ACT, true> : bwd_lean_kernel<S, KC, ACT, false>;
     hipLaunchKernelGGL(kern, dim3(g.gx, g.gy), dim3(64 * kLeanWPG), 0, st, x, dy, p.dy_stride,
                        reinterpret_cast<const uint16_t*>(a), reinterpret_cast<const uint16_t*>(b), dx,
                        part_da, part_db, p.seq, p.D, gy, g.gy1, g.n_old, g.n_total);
@@ -399,12 +405,12 @@ void bwd_layers_one(const Problem& p, const LayerOps* L, int n, hipStream_t st) 
   // launches run them: without the activation as bwd_two_pass / bwd_two_pass_r,
   // with it as bwd_two_pass_g (the dx pass then forms g for every layer, also
   // those without dx); with 64 routes the taps pass in route halves
-  constexpr bool kTwoG = ACT == 1 && bwd_two_pass_g(S, KC, true, true);
-  constexpr bool kTwo = (ACT == 0 && (bwd_two_pass(S, KC, false, true) ||
+  constexpr bool kLean = bwd_lean(S, KC, ACT != 0, true);
+  constexpr bool kTwoG = !kLean && ACT == 1 && bwd_two_pass_g(S, KC, true, true);
+  constexpr bool kTwo = (!kLean && ACT == 0 && (bwd_two_pass(S, KC, false, true) ||
                                       bwd_two_pass_r(S, KC, false, true))) ||
                         kTwoG;
   constexpr int kParts = kTwo ? taps_route_parts(KC) : 1;
-  constexpr bool kLean = MOC_BWD_LEAN && !kTwo && bwd_lean(S, KC, true);
   constexpr bool kTiers = !kTwo && !kSplit && kBwdMinWaves<S, KC, kBwdFused, true> == 2;
   const int n_cu = device_cu_count();
   // each layer's grid as bwd_one forms it (the taps pass has its own)
@@ -414,7 +420,7 @@ void bwd_layers_one(const Problem& p, const LayerOps* L, int n, hipStream_t st) 
   bool any_dx = false;
   for (int i = 0; i < n; ++i) {
     const int64_t gx_l = cdiv(L[i].D, kBwdCW);
-    const Grid2 g = kLean    ? bwd_lean_grid(p.n_tokens, gx_l, L[i].D, S, n_cu)
+    const Grid2 g = kLean    ? bwd_lean_grid(p.n_tokens, gx_l, L[i].D, S, KC, n_cu)
                     : kTiers ? bwd_grid_tiered(p.n_tokens, gx_l, L[i].D, S, n_cu)
                              : bwd_grid(p.n_tokens, L[i].D, S);
     ly.l[i] = BwdLayer{L[i].x, L[i].dy, L[i].dys, L[i].a_c, L[i].b_c, L[i].dx, L[i].part_da,
@@ -424,7 +430,7 @@ void bwd_layers_one(const Problem& p, const LayerOps* L, int n, hipStream_t st) 
     const int64_t tiles = static_cast<int64_t>(g.gx) * g.gy;
     // the dx pass of the two-pass form without the activation skips layers
     // without dx (no blocks: layer_index then never selects them)
-    blk += kSplit && !kTwo ? 8 * KC * cdiv(tiles, 8)
+    blk += kSplit && !kTwo && !kLean ? 8 * KC * cdiv(tiles, 8)
                            : (kTwo && !kTwoG && L[i].dx == nullptr ? 0 : tiles);
     any_dx = any_dx || L[i].dx != nullptr;
     if constexpr (kTwo) {
@@ -454,10 +460,10 @@ void bwd_layers_one(const Problem& p, const LayerOps* L, int n, hipStream_t st) 
     bool all_one = true;
     for (int i = 0; i < n; ++i) all_one = all_one && L[i].dys < 0;
     if (all_one)
-      hipLaunchKernelGGL((bwd_lean_layers_kernel<S, ACT, true>), dim3(static_cast<unsigned>(blk)),
+      hipLaunchKernelGGL((bwd_lean_layers_kernel<S, KC, ACT, true>), dim3(static_cast<unsigned>(blk)),
                          dim3(64 * kLeanWPG), 0, st, ly, p.seq);
     else
-      hipLaunchKernelGGL((bwd_lean_layers_kernel<S, ACT, false>), dim3(static_cast<unsigned>(blk)),
+      hipLaunchKernelGGL((bwd_lean_layers_kernel<S, KC, ACT, false>), dim3(static_cast<unsigned>(blk)),
                          dim3(64 * kLeanWPG), 0, st, ly, p.seq);
   } else {
     hipLaunchKernelGGL((bwd_layers_kernel<S, KC, kBwdNB, kBwdNC, kBwdWPG, ACT, true, kSplit, kBwdFused>),

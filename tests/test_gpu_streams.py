@@ -1,4 +1,4 @@
-"""The stream form of the fused backward (2 to 4 taps, up to 16 routes, bf16):
+"""The stream form of the fused backward (2 to 8 taps, up to 32 routes, bf16):
 ranges of one and of several steps, token counts around a step and a range, a
 ragged last channel group, segment starts at every place of a stream (between
 streams, steps and ranges included), against the oracle."""
@@ -33,7 +33,9 @@ def _check(x, a, b, dy, act, lengths=None):
         assert_close(n, u, r, BF)
 
 
-@pytest.mark.parametrize("S,K,act", [(2, 16, "silu"), (3, 7, None), (4, 16, "silu")])
+@pytest.mark.parametrize("S,K,act", [(2, 16, "silu"), (3, 7, None), (4, 16, "silu"), (4, 32, None),
+                                     (5, 12, None), (6, 20, "silu"), (7, 16, "silu"), (8, 32, "silu"),
+                                     (8, 17, None)])
 @pytest.mark.parametrize("B,T,D", [(1, 1, 2), (1, 28, 16), (1, 29, 18), (1, 30, 126), (1, 32, 128),
                                    (2, 33, 130), (1, 64, 254), (3, 5, 66)])
 def test_stream_edges_fixed(S, K, act, B, T, D):
@@ -42,12 +44,15 @@ def test_stream_edges_fixed(S, K, act, B, T, D):
            randn(g, K, S, D, scale=0.3), randn(g, B, T, D), act)
 
 
-@pytest.mark.parametrize("S,act", [(2, None), (3, "silu"), (4, "silu"), (4, None)])
+@pytest.mark.parametrize("S,K,act", [(2, 12, None), (3, 12, "silu"), (4, 12, "silu"), (4, 12, None),
+                                     (4, 32, "silu"), (6, 16, "silu"), (7, 32, None), (8, 16, "silu"),
+                                     (8, 32, None)])
 @pytest.mark.parametrize("longest", [3, 45, 700])
-def test_stream_ranges_packed(S, act, longest):
-    # 256 ranges of the two 128-channel groups; two and three steps each
+def test_stream_ranges_packed(S, K, act, longest):
+    # 256 ranges (128 of the two-wave form) of the two 128-channel groups; two to
+    # five steps each
     g = gen(S * 10 + longest)
-    N, D, K = 256 * 29 * 2 + 77, 130, 12
+    N, D = 256 * 29 * 2 + 77, 130
     lengths, left = [], N
     while left:
         n = min(left, int(torch.randint(1, longest + 1, (1,), generator=g)))
@@ -58,9 +63,10 @@ def test_stream_ranges_packed(S, act, longest):
 
 
 @pytest.mark.parametrize("form", ["one", "row"])
-def test_stream_broadcast_dy(form):
+@pytest.mark.parametrize("S,K", [(4, 16), (8, 32), (7, 8)])
+def test_stream_broadcast_dy(form, S, K):
     g = gen(7)
-    B, T, D, K, S = 1, 256 * 29 + 1, 258, 16, 4
+    B, T, D = 1, 256 * 29 + 1, 258
     dy = randn(g, 1, 1, 1) if form == "one" else randn(g, 1, 1, D)
     _check(randn(g, B, T, D, scale=0.5), torch.softmax(randn(g, B, T, K), -1),
            randn(g, K, S, D, scale=0.3), dy, "silu")
