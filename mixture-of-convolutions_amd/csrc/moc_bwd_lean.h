@@ -1,4 +1,4 @@
-// Fused backward (stage 1) of bf16 layers with 2 to 8 taps and up to 32 routes.
+// Fused backward (stage 1) with 2 to 8 taps: bf16 up to 32 routes, fp32 up to 16.
 //
 // What bounds it: instruction issue and the latency chains of two to four waves
 // per SIMD (four, 128 VGPRs, with 2 to 4 taps and 16 routes; else two, 256 VGPRs).
@@ -27,7 +27,18 @@
 //   32 routes  94.5->82.9       127->94          130->102         161->129         194.6->158
 //              116->85.7        152->95.5        190->109         217->137         252->169
 // and D 4096: 32768 tokens, 16 routes, 4 taps 275 -> 262.6; 16384 tokens, 32
-// routes, 8 taps 335 -> 280.  So it serves every shape it is built for.
+// routes, 8 taps 335 -> 280.  So it serves every bf16 shape it is built for.
+//
+// fp32 (every product on v_mfma_f32_16x16x4_f32, whose rate is half of what bounds
+// it: 96 of them, 3072 cycles, a step and wave at 4 taps, 82 us of the 165 below;
+// m needs no split, and its dbasis operand is the lane's own registers).  Backward
+// entry, B4 T4096 D2048, 16 routes, without / with SiLU, us, the fused pass of
+// bwd_tile or the two passes with g through memory -> here:
+//   taps  2            3            4            5            6            8
+//         111->(114)   170->132     206->158     249->184     260->209     330->263
+//         132->118     180->137     273->165     342->193     352->223     484->282
+// B4 T2048 D1024, 4 taps, SiLU: 92 -> 54, its training step 145 -> 108; same
+// order at 4 routes, D 4096, and 600 rows of D 3000.
 //
 // Work per step and wave (rows 8 i .. 8 i + 7 of each stream):
 //   W_s = alpha . basis_s by MFMA (16x16x16, or 16x16x32 over 32 routes; both
@@ -72,21 +83,32 @@ struct TrTile1 {
   }
 };
 
-__device__ __forceinline__ f32x4 mma16(s16x4 a, s16x4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-}
-
 constexpr int kLeanWPG = 8;        // waves per workgroup (8 x 16 = 128 channels)
 constexpr int kLeanCW = 16;        // channels per wave
 
-// Shapes the lean pass serves (bf16 operands).
+// Shapes the lean pass serves (fp32 with 2 taps and no activation, where there is
+// little to form or share: 111 us in the fused pass of bwd_tile, 114 here)
 constexpr bool bwd_lean(int S, int KC, bool act, bool bf) {
-  return bf && KC <= 2 && S >= 2 && S <= 8;
+  return KC <= (bf ? 2 : 1) && S >= 2 && S <= 8 && (bf || act || S > 2);
 }
 // Waves per SIMD it is built for: four (128 VGPRs, two workgroups per CU) with 2
-// to 4 taps and 16 routes, else two (256 VGPRs and up to 156 KB of LDS, one
-// workgroup per CU)
-constexpr int lean_waves(int S, int KC) { return S <= 4 && KC == 1 ? 4 : 2; }
+// to 4 taps and 16 routes in bf16, else two (256 VGPRs and up to 156 KB of LDS,
+// one workgroup per CU)
+constexpr int lean_waves(int S, int KC, bool bf = true) { return bf && S <= 4 && KC == 1 ? 4 : 2; }
+
+// LDS tiles of the fp32 form: rows of 16 floats, the 4-float chunk c of row r at
+// chunk c ^ sw, and 16 floats of padding after every P rows.  Tiles that 16
+// lanes read 16 bytes each down 16 rows, and that the wave writes or reads a
+// float per lane across four row groups P apart, touch every bank once.
+template <int P>
+__device__ __forceinline__ int f32_slot(int row, int chunk, int sw) {
+  return row * 16 + (row / P) * 16 + 4 * (chunk ^ sw);
+}
+// routing weights (rows 8 q + r), m (likewise) and the basis (routes)
+__device__ __forceinline__ int f32_aslot(int row, int chunk) { return f32_slot<8>(row, chunk, row >> 3); }
+__device__ __forceinline__ int f32_mslot(int row, int chunk) { return f32_slot<8>(row, chunk, (row >> 2) & 3); }
+__device__ __forceinline__ int f32_bslot(int row, int chunk) { return f32_slot<4>(row, chunk, row >> 2); }
+constexpr int kF32Rows = 32 * 16 + 3 * 16, kF32Basis = 16 * 16 + 3 * 16;  // floats of a tile
 
 // Rows of a row-major tensor walked with the scalar unit: next(bytes) is a buffer
 // from the current row on (`left` bytes; at most 0 past the end: loads give
@@ -108,28 +130,30 @@ struct RowWalk {
 
 // The work of workgroup (bx, by) of one layer; the __global__ wrappers below
 // map a single launch's 2-D grid or a grouped launch's 1-D grid onto it.
-template <int S, int KC, int ACT, bool DY1>
+template <int S, int KC, int ACT, bool DY1, bool BF>
 __device__ __forceinline__ void
 bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t dys,
-              const uint16_t* __restrict__ a_c, const uint16_t* __restrict__ b_c,
-              void* __restrict__ dxv, float* __restrict__ part_da, float* __restrict__ part_db,
+              const typename CT<BF>::elem* __restrict__ a_c,
+              const typename CT<BF>::elem* __restrict__ b_c, void* __restrict__ dxv, float* __restrict__ part_da, float* __restrict__ part_db,
               SeqLayout seq, int64_t D, int bx, int by, int gy, int gy1, int n_old, int n_total,
               bool act_rt = false) {
   const bool act = ACT == kActRuntime ? act_rt : ACT != 0;  // (uniform)
-  using E = uint16_t;
-  using Op = s16x4;
+  using C = CT<BF>;
+  using E = typename C::elem;
+  using Op = typename C::opnd;
   constexpr int NB = 2, R = 8, TB = 32, H = S - 1, W = R + H;
   constexpr int KP = 16 * KC, WPG = kLeanWPG, CW = kLeanCW;
-  constexpr int ESZ = 2;
+  constexpr int ESZ = sizeof(E);
   static_assert(S >= 2 && S <= 8 && KC <= 2, "lean backward: 2 to 8 taps, up to 32 routes");
+  static_assert(BF || KC == 1, "fp32: up to 16 routes");
   // the four-wave form leaves what a stream owes its predecessor in LDS
-  constexpr bool kC0Lds = lean_waves(S, KC) == 4;
+  constexpr bool kC0Lds = lean_waves(S, KC, BF) == 4;
   // The next step's rows are loaded where this step's have been converted in the
   // two-wave form (a SIMD has one other wave to cover the loads: 16 routes, 8
   // taps 80.9 -> 77.1 us, 32 routes, 4 taps 115.4 -> 109.0), after the m products
   // in the others (four waves cover them; 8 taps with 32 routes would spill, 167
   // -> 204 us)
-  constexpr bool kFetchEarly = lean_waves(S, KC) == 2 && !(S == 8 && KC == 2);
+  constexpr bool kFetchEarly = lean_waves(S, KC, BF) == 2 && !(S == 8 && KC == 2);
 
   // routing-weight rows of a step, unpadded: row rho = 8 q + r is row r of
   // stream q; the 8-byte chunk c (4 routes) of row rho sits at chunk c ^ asw(rho)
@@ -137,11 +161,12 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
   auto asw = [](int row) -> int {
     return KC == 1 ? (row >> 3) & 3 : ((row >> 1) & 1) | (((row >> 3) & 3) << 1);
   };
-  __shared__ __align__(16) E a_lds[2][TB][KP];
-  __shared__ __align__(16) Op m_tr[WPG][2][TrTile1::kSlots];  // [wave][hi / lo]
+  __shared__ __align__(16) E a_lds[2][BF ? TB : 1][BF ? KP : kF32Rows];
+  __shared__ __align__(16) Op m_tr[BF ? WPG : 1][2][TrTile1::kSlots];  // [wave][hi / lo]
+  __shared__ __align__(16) float m_f32[BF ? 1 : WPG][kF32Rows];        // fp32: rows x channels
   // basis tile of each wave, b_lds[wave][s][kc][route j][4 channels, chunk q ^
   // (j / 4)] (a 16-lane group of a read touches 16 distinct slots)
-  __shared__ __align__(16) Op b_lds[WPG][S][KC][16 * 4];
+  __shared__ __align__(16) Op b_lds[WPG][S][KC][BF ? 16 * 4 : kF32Basis / 4];
   __shared__ float da_lds[2][WPG][NB][KC][16][17];
   __shared__ float c0_lds[kC0Lds ? H : 1][kC0Lds ? 64 * WPG : 1];
 
@@ -189,7 +214,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
   if constexpr (DY1) {
     E e;
     Buf(dyv, ESZ).load<ESZ>(ch_ok ? 0u : kOffNone, &e);
-    dy1 = bf16_to_f32(e);
+    dy1 = C::to_f(e);
   }
   const Buf bb(b_c, static_cast<int64_t>(KP) * S * D * ESZ);
 
@@ -204,12 +229,12 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc) {
         Op bda;
-        bb.load<8>(row_off((16 * kc + j) * S + s, 0, rb, static_cast<uint32_t>(ch * ESZ), on), &bda);
+        bb.load<4 * ESZ>(row_off((16 * kc + j) * S + s, 0, rb, static_cast<uint32_t>(ch * ESZ), on), &bda);
         if (ch + 2 >= D) {
           bda[2] = 0;
           bda[3] = 0;
         }
-        b_lds[wave][s][kc][j * 4 + (q ^ (j >> 2))] = bda;
+        b_lds[wave][s][kc][BF ? j * 4 + (q ^ (j >> 2)) : f32_bslot(j, q) / 4] = bda;
       }
   }
   f32x4 dbacc[S][KC];
@@ -237,7 +262,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
       }
     }
   };
-  // routing-weight rows of a step: 32 rows, 8 bytes per thread of the first 2 KC
+  // routing-weight rows of a step: 32 rows, 4 routes per thread of the first 2 KC
   // waves (row rho: thread 4 KC rho + chunk)
   // (the per-lane terms are formed where they are used, from an opaque copy of
   // the thread id: hoisted out of the loop they outgrow the register budget)
@@ -253,13 +278,15 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
     const Buf ab = aw.next(R * KP * ESZ);
     if (wave < 2 * KC) {
       const int t = opaque_tid(), row = t / (4 * KC);
-      ab.load<8>(static_cast<uint32_t>((R * n * (row >> 3) + (row & 7)) * KP * ESZ + (t % (4 * KC)) * 8), arw);
+      ab.load<4 * ESZ>(static_cast<uint32_t>(((R * n * (row >> 3) + (row & 7)) * KP + (t % (4 * KC)) * 4) * ESZ),
+                       arw);
     }
   };
   auto stage_alpha = [&](int buf) {
     if (wave < 2 * KC) {
       const int t = opaque_tid(), row = t / (4 * KC);
-      Vec<E, 4>::store(&a_lds[buf][row][((t % (4 * KC)) ^ asw(row)) * 4], arw);
+      if constexpr (BF) Vec<E, 4>::store(&a_lds[buf][row][((t % (4 * KC)) ^ asw(row)) * 4], arw);
+      else Vec<E, 4>::store(&a_lds[buf][0][f32_aslot(row, t % 4)], arw);
     }
   };
 
@@ -271,7 +298,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
     E e;
     const int64_t lo = first - H > 0 ? first - H : 0;
     Buf(static_cast<const char*>(xv) + lo * rb, (row_hi - lo) * rb).load<ESZ>(row_off(u, lo, rb, col, ch_ok), &e);
-    xw[R + w] = bf16_to_f32(e);
+    xw[R + w] = C::to_f(e);
   }
   fetch_xdy();
   fetch_a();
@@ -312,8 +339,8 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
     float g[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      xw[H + r] = bf16_to_f32(xr[r]);
-      g[r] = DY1 ? dy1 : bf16_to_f32(dr[DY1 ? 0 : r]);
+      xw[H + r] = C::to_f(xr[r]);
+      g[r] = DY1 ? dy1 : C::to_f(dr[DY1 ? 0 : r]);
     }
     // (unconditionally, also after the last step: rows past the buffer load zeros)
     fetch_a();
@@ -330,7 +357,10 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc) {
         const int row = R * (j >> 2) + 4 * b + (j & 3);
-        aop[b][kc] = *reinterpret_cast<const Op*>(&a_lds[buf][row][((4 * kc + q) ^ asw(row)) * 4]);
+        if constexpr (BF)
+          aop[b][kc] = *reinterpret_cast<const Op*>(&a_lds[buf][row][((4 * kc + q) ^ asw(row)) * 4]);
+        else
+          aop[b][kc] = *reinterpret_cast<const Op*>(&a_lds[buf][0][f32_aslot(row, q)]);
       }
 
     f32x4 dacc[NB][KC];
@@ -374,13 +404,20 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
       auto form_w = [&](int s, f32x4 (&w)[NB]) {
         Op bop[KC];
 #pragma unroll
-        for (int kc = 0; kc < KC; ++kc)
-          bop[kc] = TrTile<NB, 2>::read(&b_lds[wave][s][kc][(4 * q + (j >> 2)) * 4 + ((j & 3) ^ q)]);
+        for (int kc = 0; kc < KC; ++kc) {
+          if constexpr (BF) {
+            bop[kc] = TrTile<NB, 2>::read(&b_lds[wave][s][kc][(4 * q + (j >> 2)) * 4 + ((j & 3) ^ q)]);
+          } else {
+            const float* bt = reinterpret_cast<const float*>(&b_lds[wave][s][kc][0]);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) bop[kc][v] = bt[f32_bslot(4 * q + v, j >> 2) + (j & 3)];
+          }
+        }
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
           const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
           if constexpr (KC == 2) w[b] = mma32(aop[b][0], aop[b][1], bop[0], bop[1], zero);
-          else w[b] = mma16(aop[b][0], bop[0], zero);
+          else w[b] = C::mma(aop[b][0], bop[0], zero);
         }
       };
       constexpr bool kKeepW = ACT != 0 || KC == 1;
@@ -435,82 +472,121 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
         // they belong to the stream (or range) before
 #pragma unroll
         for (int w = 0; w < R; ++w) {
-          const E o = f32_to_bf16(dxa[w]);
+          const E o = C::from_f(dxa[w]);
           dxw.next(rb, w >= H || i > 0).store<ESZ>(vx, &o);
         }
       }
 
       // alpha^T operands of the dbasis MFMA, own rows only (the last step's
       // final S-1 rows of stream 3 are the next range's; rows past N are zero):
-      // at[b] = alpha[row 8 q + 4 b + v, j] (transposed read of the staged rows)
+      // at[b][v] = alpha[row 8 q + 4 b + v, j] (transposed read of the staged rows)
       Op at[NB][KC];
 #pragma unroll
       for (int b = 0; b < NB; ++b)
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) {
           const int row = R * q + 4 * b + (j >> 2);
-          at[b][kc] = TrTile<NB, 2>::read(&a_lds[buf][row][((4 * kc + (j & 3)) ^ asw(row)) * 4]);
+          if constexpr (BF) {
+            at[b][kc] = TrTile<NB, 2>::read(&a_lds[buf][row][((4 * kc + (j & 3)) ^ asw(row)) * 4]);
+          } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              at[b][kc][v] = a_lds[buf][0][f32_aslot(R * q + 4 * b + v, j >> 2) + (j & 3)];
+          }
         }
       if (!more) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
           constexpr int kOwn = R - H;  // rows of stream 3 that are still this range's
           const int n_ok = kOwn - 4 * b < 0 ? 0 : (kOwn - 4 * b < 4 ? kOwn - 4 * b : 4);
-          const uint64_t keep = q == 3 && n_ok < 4 ? ((1ull << (16 * n_ok)) - 1ull) : ~0ull;
+          if constexpr (BF) {
+            const uint64_t keep = q == 3 && n_ok < 4 ? ((1ull << (16 * n_ok)) - 1ull) : ~0ull;
 #pragma unroll
-          for (int kc = 0; kc < KC; ++kc)
-            at[b][kc] = __builtin_bit_cast(Op, __builtin_bit_cast(uint64_t, at[b][kc]) & keep);
+            for (int kc = 0; kc < KC; ++kc)
+              at[b][kc] = __builtin_bit_cast(Op, __builtin_bit_cast(uint64_t, at[b][kc]) & keep);
+          } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              if (q == 3 && v >= n_ok) at[b][0][v] = 0.f;
+          }
         }
       }
-      // m of tap s -> hi / lo operands -> this wave's tile, dbasis MFMAs
-      auto stage_m = [&](int s) {
-        Op mh[NB], ml[NB];
+      if constexpr (BF) {
+        // m of tap s -> hi / lo operands -> this wave's tile, dbasis MFMAs
+        auto stage_m = [&](int s) {
+          Op mh[NB], ml[NB];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          uint32_t hbits[4];
-          float lo[4];
+          for (int b = 0; b < NB; ++b) {
+            uint32_t hbits[4];
+            float lo[4];
 #pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int r = 4 * b + v;
-            const float mval = tap_ok(r, s) ? g[r] * xw[r + s] : 0.f;
-            hbits[v] = __float_as_uint(mval) & 0xffff0000u;
-            lo[v] = mval - __uint_as_float(hbits[v]);
+            for (int v = 0; v < 4; ++v) {
+              const int r = 4 * b + v;
+              const float mval = tap_ok(r, s) ? g[r] * xw[r + s] : 0.f;
+              hbits[v] = __float_as_uint(mval) & 0xffff0000u;
+              lo[v] = mval - __uint_as_float(hbits[v]);
+            }
+            mh[b] = pack4_hi(hbits[0], hbits[1], hbits[2], hbits[3]);
+            ml[b] = pack4_bf16(lo[0], lo[1], lo[2], lo[3]);
+            m_tr[wave][0][TrTile1::wslot(j, q, b)] = mh[b];
+            m_tr[wave][1][TrTile1::wslot(j, q, b)] = ml[b];
           }
-          mh[b] = pack4_hi(hbits[0], hbits[1], hbits[2], hbits[3]);
-          ml[b] = pack4_bf16(lo[0], lo[1], lo[2], lo[3]);
-          m_tr[wave][0][TrTile1::wslot(j, q, b)] = mh[b];
-          m_tr[wave][1][TrTile1::wslot(j, q, b)] = ml[b];
+#pragma unroll
+          for (int kc = 0; kc < KC; ++kc) {
+            dbacc[s][kc] = mma32(mh[0], mh[1], at[0][kc], at[1][kc], dbacc[s][kc]);
+            dbacc[s][kc] = mma32(ml[0], ml[1], at[0][kc], at[1][kc], dbacc[s][kc]);
+          }
+        };
+        // dalpha contracts 16 channels of the hi and of the lo part in one
+        // 16x16x32 MFMA against the basis operand twice.  The transposed reads of
+        // a tap (ra[rb][h] = m[16 rb + i][4 qq + {0..3}]) are issued before the next
+        // tap's m values are formed and written (a wave's LDS operations complete
+        // in issue order, so one tile serves)
+        Op ra[NB][2], bda[KC];
+        stage_m(0);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+          wave_lds_sync();
+#pragma unroll
+          for (int r2 = 0; r2 < NB; ++r2)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+              ra[r2][h] = TrTile<NB, 2>::read(&m_tr[wave][h][TrTile1::rslot(j, q, r2)]);
+#pragma unroll
+          for (int kc = 0; kc < KC; ++kc) bda[kc] = b_lds[wave][s][kc][j * 4 + (q ^ (j >> 2))];
+          __builtin_amdgcn_sched_barrier(0);
+          if (s + 1 < S) stage_m(s + 1);
+#pragma unroll
+          for (int r2 = 0; r2 < NB; ++r2)
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc)
+              dacc[r2][kc] = mma32(ra[r2][0], ra[r2][1], bda[kc], bda[kc], dacc[r2][kc]);
         }
+      } else {
+        // fp32: m is the dbasis A operand as it lies (row r of every stream in
+        // one 16x16x4 product), its transpose for dalpha goes through the tile
+        auto stage_m = [&](int s) {
 #pragma unroll
-        for (int kc = 0; kc < KC; ++kc) {
-          dbacc[s][kc] = mma32(mh[0], mh[1], at[0][kc], at[1][kc], dbacc[s][kc]);
-          dbacc[s][kc] = mma32(ml[0], ml[1], at[0][kc], at[1][kc], dbacc[s][kc]);
+          for (int r = 0; r < R; ++r) {
+            const float mval = tap_ok(r, s) ? g[r] * xw[r + s] : 0.f;
+            m_f32[wave][f32_mslot(R * q + r, j >> 2) + (j & 3)] = mval;
+            dbacc[s][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(mval, at[r >> 2][0][r & 3], dbacc[s][0], 0, 0, 0);
+          }
+        };
+        Op ra[NB], bda;
+        stage_m(0);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+          wave_lds_sync();
+#pragma unroll
+          for (int r2 = 0; r2 < NB; ++r2)
+            ra[r2] = *reinterpret_cast<const Op*>(&m_f32[wave][f32_mslot(16 * r2 + j, q)]);
+          bda = b_lds[wave][s][0][f32_bslot(j, q) / 4];
+          __builtin_amdgcn_sched_barrier(0);
+          if (s + 1 < S) stage_m(s + 1);
+#pragma unroll
+          for (int r2 = 0; r2 < NB; ++r2) dacc[r2][0] = C::mma(ra[r2], bda, dacc[r2][0]);
         }
-      };
-      // dalpha contracts 16 channels of the hi and of the lo part in one
-      // 16x16x32 MFMA against the basis operand twice.  The transposed reads of
-      // a tap (ra[rb][h] = m[16 rb + i][4 qq + {0..3}]) are issued before the next
-      // tap's m values are formed and written (a wave's LDS operations complete
-      // in issue order, so one tile serves)
-      Op ra[NB][2], bda[KC];
-      stage_m(0);
-#pragma unroll
-      for (int s = 0; s < S; ++s) {
-        wave_lds_sync();
-#pragma unroll
-        for (int r2 = 0; r2 < NB; ++r2)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            ra[r2][h] = TrTile<NB, 2>::read(&m_tr[wave][h][TrTile1::rslot(j, q, r2)]);
-#pragma unroll
-        for (int kc = 0; kc < KC; ++kc) bda[kc] = b_lds[wave][s][kc][j * 4 + (q ^ (j >> 2))];
-        __builtin_amdgcn_sched_barrier(0);
-        if (s + 1 < S) stage_m(s + 1);
-#pragma unroll
-        for (int r2 = 0; r2 < NB; ++r2)
-#pragma unroll
-          for (int kc = 0; kc < KC; ++kc)
-            dacc[r2][kc] = mma32(ra[r2][0], ra[r2][1], bda[kc], bda[kc], dacc[r2][kc]);
       }
       wave_lds_sync();
     }
@@ -560,7 +636,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
     for (int e = 0; e < H; ++e) {
       const int from = (lane + 16) & 63;
       const float owed = kC0Lds ? c0_lds[kC0Lds ? e : 0][kC0Lds ? (tid & ~63) | from : 0] : __shfl(c0[e], from, 64);
-      const E o = f32_to_bf16(dxa[R + e] + owed);
+      const E o = C::from_f(dxa[R + e] + owed);
       dxw.next(rb).store<ESZ>(vx, &o);
     }
   }
@@ -586,13 +662,13 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
   }
 }
 
-template <int S, int KC, bool ACT, bool DY1>
-__global__ void __launch_bounds__(64 * kLeanWPG) __attribute__((amdgpu_waves_per_eu(lean_waves(S, KC))))
+template <int S, int KC, bool ACT, bool DY1, bool BF>
+__global__ void __launch_bounds__(64 * kLeanWPG) __attribute__((amdgpu_waves_per_eu(lean_waves(S, KC, BF))))
 bwd_lean_kernel(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t dys,
-                const uint16_t* __restrict__ a_c, const uint16_t* __restrict__ b_c,
-                void* __restrict__ dxv, float* __restrict__ part_da, float* __restrict__ part_db,
+                const typename CT<BF>::elem* __restrict__ a_c,
+                const typename CT<BF>::elem* __restrict__ b_c, void* __restrict__ dxv, float* __restrict__ part_da, float* __restrict__ part_db,
                 SeqLayout seq, int64_t D, int gy, int gy1, int n_old, int n_total) {
-  bwd_lean_tile<S, KC, ACT, DY1>(xv, dyv, dys, a_c, b_c, dxv, part_da, part_db, seq, D,
+  bwd_lean_tile<S, KC, ACT, DY1, BF>(xv, dyv, dys, a_c, b_c, dxv, part_da, part_db, seq, D,
                         static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), gy, gy1, n_old,
                         n_total);
 }
@@ -611,7 +687,7 @@ bwd_lean_layers_kernel(BwdLayers ly, SeqLayout seq) {
     local -= gxl;
     ++row;
   }
-  bwd_lean_tile<S, KC, ACT, DY1>(Lp->x, Lp->dy, Lp->dys, static_cast<const uint16_t*>(Lp->a),
+  bwd_lean_tile<S, KC, ACT, DY1, true>(Lp->x, Lp->dy, Lp->dys, static_cast<const uint16_t*>(Lp->a),
                         static_cast<const uint16_t*>(Lp->b), Lp->dx, Lp->part_da, Lp->part_db, seq,
                         Lp->D, local, row, Lp->gy, Lp->gy1, Lp->n_old, Lp->n_total, Lp->act != 0);
 }

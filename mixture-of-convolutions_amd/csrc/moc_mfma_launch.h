@@ -249,8 +249,8 @@ inline Grid2 bwd_taps_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int n_cu
 // S - 1 in all (n steps own 32 n - (S - 1) rows; range by starts at row
 // 32 steps_before - by (S - 1)).  Every range has at least one step: there are
 // at most ceil(N / (32 - (S - 1))) ranges.
-inline Grid2 bwd_lean_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int KC, int n_cu) {
-  const bool four = lean_waves(static_cast<int>(S), KC) == 4;
+inline Grid2 bwd_lean_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int KC, bool bf, int n_cu) {
+  const bool four = lean_waves(static_cast<int>(S), KC, bf) == 4;
   Grid2 g = four ? bwd_grid_tiered(N, gx, D, S, n_cu) : bwd_taps_grid(N, gx, D, S, n_cu);
   const int64_t gy = g.gy, gy1 = g.gy1;
   const int64_t steps = cdiv(N + gy * (S - 1), 16 * kBwdNB);
@@ -270,7 +270,8 @@ inline Grid2 bwd_lean_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int KC, 
 // fused pass's.
 inline Grid2 bwd_partials_grid(const Problem& p) {
   if (bwd_lean(p))
-    return bwd_lean_grid(p.n_tokens, cdiv(p.D, kBwdCW), p.D, p.S, route_chunks(p.K), device_cu_count());
+    return bwd_lean_grid(p.n_tokens, cdiv(p.D, kBwdCW), p.D, p.S, route_chunks(p.K), p.x_dt == DT_BF16,
+                         device_cu_count());
   return bwd_two_pass(p) ? bwd_taps_grid(p.n_tokens, cdiv(p.D, kTapsCW), p.D, p.S,
                                          device_cu_count() / taps_route_parts(route_chunks(p.K)))
                          : bwd_grid_gx(p.n_tokens, cdiv(p.D, kBwdCW), p.D, p.S);
@@ -324,7 +325,7 @@ void bwd_one(const Problem& p, const void* x, const void* dy, const void* a_c, c
   // tiers for the fused pass at two resident workgroups per CU (not split in route chunks)
   constexpr bool kTiers = !kTwo && !kSplit && kBwdMinWaves<S, KC, kBwdFused, BF> == 2;
   const int64_t gx_all = cdiv(p.D, kBwdCW);
-  const Grid2 g = kLean    ? bwd_lean_grid(p.n_tokens, gx_all, p.D, S, KC, device_cu_count())
+  const Grid2 g = kLean    ? bwd_lean_grid(p.n_tokens, gx_all, p.D, S, KC, BF, device_cu_count())
                   : kTiers ? bwd_grid_tiered(p.n_tokens, gx_all, p.D, S, device_cu_count())
                            : bwd_grid(p.n_tokens, p.D, S);
   const auto* a = static_cast<const E*>(a_c);
@@ -355,9 +356,8 @@ void bwd_one(const Problem& p, const void* x, const void* dy, const void* a_c, c
   } else if constexpr (kLean) {
     // (the lean pass's workgroup covers the same kBwdCW channels with 8 waves)
     // (one dy element for every token and channel: its own instantiation)
-    auto kern = p.dy_stride < 0 ? bwd_lean_kernel<S, KC, ACT, true> : bwd_lean_kernel<S, KC, ACT, false>;
-    hipLaunchKernelGGL(kern, dim3(g.gx, g.gy), dim3(64 * kLeanWPG), 0, st, x, dy, p.dy_stride,
-                       reinterpret_cast<const uint16_t*>(a), reinterpret_cast<const uint16_t*>(b), dx,
+    auto kern = p.dy_stride < 0 ? bwd_lean_kernel<S, KC, ACT, true, BF> : bwd_lean_kernel<S, KC, ACT, false, BF>;
+    hipLaunchKernelGGL(kern, dim3(g.gx, g.gy), dim3(64 * kLeanWPG), 0, st, x, dy, p.dy_stride, a, b, dx,
                        part_da, part_db, p.seq, p.D, gy, g.gy1, g.n_old, g.n_total);
   } else {
     hipLaunchKernelGGL((bwd_kernel<S, KC, kBwdNB, kBwdNC, kBwdWPG, ACT, BF, kSplit, kBwdFused>),
@@ -420,7 +420,7 @@ void bwd_layers_one(const Problem& p, const LayerOps* L, int n, hipStream_t st) 
   bool any_dx = false;
   for (int i = 0; i < n; ++i) {
     const int64_t gx_l = cdiv(L[i].D, kBwdCW);
-    const Grid2 g = kLean    ? bwd_lean_grid(p.n_tokens, gx_l, L[i].D, S, KC, n_cu)
+    const Grid2 g = kLean    ? bwd_lean_grid(p.n_tokens, gx_l, L[i].D, S, KC, true, n_cu)
                     : kTiers ? bwd_grid_tiered(p.n_tokens, gx_l, L[i].D, S, n_cu)
                              : bwd_grid(p.n_tokens, L[i].D, S);
     ly.l[i] = BwdLayer{L[i].x, L[i].dy, L[i].dys, L[i].a_c, L[i].b_c, L[i].dx, L[i].part_da,
