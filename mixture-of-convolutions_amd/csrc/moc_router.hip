@@ -53,13 +53,18 @@ __device__ __forceinline__ s16x4 tr_read(const void* p) {
 }
 
 // ---------------------------------------------------------------------------
-// logits[t, k] = sum_z z[t, z] router[k, z].  Workgroup: 32 tokens (two blocks
-// of 16), 4 waves.  Wave w sums the 64-wide z chunks c = w, w + 4, ...: lane
+// logits[t, k] = sum_z z[t, z] router[k, z].  Workgroup: HB blocks of 16 tokens
+// (two; four with more than 32 routes and rows enough: below), 4 waves.  Wave w sums the 64-wide z chunks c = w, w + 4, ...: lane
 // (i, qq) loads columns 64 c + 8 qq + [0, 8) and 64 c + 32 + 8 qq + [0, 8) of
-// tokens t0 + i, t0 + 16 + i (A operands) and of route 16 kc + i (B operands),
+// tokens t0 + 16 h + i (A operands) and of route 16 kc + i (B operands),
 // so that each load instruction reads 64 contiguous bytes per row and the
-// router operands serve both token blocks.  The 4 partial tiles are summed in
+// router operands serve every token block.  The 4 partial tiles are summed in
 // LDS in wave order.
+// Two token blocks re-read the whole router from L2 for every 32 rows of z (96
+// routes, Z 4096: 402 MB of it beside 134 MB of z at N 16384, 67 us); four halve
+// that (45.5 us), a wave per SIMD with up to 256 VGPRs holding the next round's
+// loads.  Up to 32 routes the router is the smaller part, and below 64 x 256
+// rows (one workgroup for each of 256 CUs) the smaller workgroups fill the chip.
 // Chunks whose loads are issued together: four up to 32 routes, fewer above
 // (the router operands of a chunk take 8 KC registers per lane).
 template <int KC>
@@ -98,34 +103,34 @@ __device__ __forceinline__ void route_group(float (&l)[32], int kn, int routing)
   }
 }
 
-template <int KC, bool GROUPED>
+template <int KC, bool GROUPED, int HB>
 __global__ void __launch_bounds__(256) router_fwd_kernel(const uint16_t* __restrict__ z,
                                                          const uint16_t* __restrict__ r,
                                                          uint16_t* __restrict__ logits,
                                                          int64_t N, int Z, int K, int routing,
                                                          RouteGroups grp) {
   constexpr int KP = 16 * KC;
-  constexpr int UB = kFwdBatch<KC>;
-  __shared__ float red[4][2][KP][17];
+  constexpr int UB = kFwdBatch<KC>, TOK = 16 * HB;
+  __shared__ float red[4][HB][KP][17];
   const int lane = threadIdx.x & 63, w = wave_id();
   const int i = lane & 15, qq = lane >> 4;
-  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 32;
-  const int64_t rows = (N - t0 < 32) ? N - t0 : 32;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * TOK;
+  const int64_t rows = (N - t0 < TOK) ? N - t0 : TOK;
   // rows past N and routes past K lie outside the buffers and load zeros
   const Buf zb(z + t0 * Z, rows * Z * 2);
   const Buf rb(r, static_cast<int64_t>(K) * Z * 2);
-  f32x4 acc[2][KC];
+  f32x4 acc[HB][KC];
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int h = 0; h < HB; ++h)
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) acc[h][kc] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int nchunk = Z / 64;
   // UB chunks per round (4 + 2 KC loads per chunk and lane).  Above 32 routes
   // (rounds of one or two chunks) two rounds are in flight: the loads of round
   // r + 1 are issued before the MFMAs of round r (two register sets, the loop
-  // unrolled by two so that neither is copied; grouped router of configs[4]:
+  // unrolled by two so that neither is copied; grouped router of N 16384, Z 4096, 96 routes:
   // 89 -> 81 us).  Chunks past the row end load zeros instead of branching.
-  typedef u32x4 ZOps[UB][2][2];
+  typedef u32x4 ZOps[UB][HB][2];
   typedef u32x4 ROps[UB][KC][2];
   auto load_round = [&](int c0, ZOps& za, ROps& ra) {
 #pragma unroll
@@ -134,7 +139,7 @@ __global__ void __launch_bounds__(256) router_fwd_kernel(const uint16_t* __restr
       const bool on = c < nchunk;
       const uint32_t col0 = static_cast<uint32_t>((64 * c + 8 * qq) * 2), col1 = col0 + 64;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < HB; ++h) {
         const uint32_t zrow = static_cast<uint32_t>((16 * h + i) * Z * 2);
         za[u][h][0] = load16(zb, on ? zrow + col0 : kOffNone);
         za[u][h][1] = load16(zb, on ? zrow + col1 : kOffNone);
@@ -153,7 +158,7 @@ __global__ void __launch_bounds__(256) router_fwd_kernel(const uint16_t* __restr
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < HB; ++h) {
           acc[h][kc] = mma8(za[u][h][0], ra[u][kc][0], acc[h][kc]);
           acc[h][kc] = mma8(za[u][h][1], ra[u][kc][1], acc[h][kc]);
         }
@@ -183,7 +188,7 @@ __global__ void __launch_bounds__(256) router_fwd_kernel(const uint16_t* __restr
   }
   // D lane (j, q): route 16 kc + j, tokens 16 h + 4 q + v
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int h = 0; h < HB; ++h)
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
@@ -191,8 +196,8 @@ __global__ void __launch_bounds__(256) router_fwd_kernel(const uint16_t* __restr
   __syncthreads();
   if constexpr (GROUPED) {
     // route groups: one thread per (group, token) forms the group's weights
-    for (int idx = threadIdx.x; idx < 32 * grp.n; idx += 256) {
-      const int tok = idx & 31, gi = idx >> 5, h = tok >> 4, tr = tok & 15;
+    for (int idx = threadIdx.x; idx < TOK * grp.n; idx += 256) {
+      const int tok = idx % TOK, gi = idx / TOK, h = tok >> 4, tr = tok & 15;
       if (tok >= rows) continue;
       const int k0 = grp.k0[gi], kn = grp.kn[gi];
       float l[32];
@@ -219,7 +224,7 @@ __global__ void __launch_bounds__(256) router_fwd_kernel(const uint16_t* __restr
   // KP consecutive lanes hold one token's routes; every lane runs every pass
   // (the shuffles of the routing need all of them; routing needs KC <= 2)
 #pragma unroll
-  for (int pass = 0; pass < 32 * KP / 256; ++pass) {
+  for (int pass = 0; pass < TOK * KP / 256; ++pass) {
     const int idx = threadIdx.x + 256 * pass;
     const int tok = idx / KP, k = idx % KP, h = tok >> 4, tr = tok & 15;
     const float s = ((red[0][h][k][tr] + red[1][h][k][tr]) + red[2][h][k][tr]) + red[3][h][k][tr];
@@ -472,9 +477,12 @@ __global__ void __launch_bounds__(256) router_dr_kernel(const uint16_t* __restri
 // in turn, the same block order, so the partials are the same bit for bit)
 // also writes dz for its columns and tokens, D[zc][t] = router^T . dl^T as in
 // router_dz_kernel, with the dl B operands read from the block's LDS tile.
-// Three blocks' loads are in flight per wave.
+// Three blocks' loads are in flight per wave, two above 32 routes.
+// N 16384, Z 4096, 96 routes: 94 us as router_dz_kernel and router_dr_kernel (two
+// launches, each at half the copy rate), 84 here.
 template <int KC>
-__global__ void __launch_bounds__(256) router_bwd_kernel(const uint16_t* __restrict__ dl,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KC > 2 ? 2 : 1)))
+router_bwd_kernel(const uint16_t* __restrict__ dl,
                                                          const uint16_t* __restrict__ z,
                                                          const uint16_t* __restrict__ r,
                                                          uint16_t* __restrict__ dz,
@@ -484,7 +492,12 @@ __global__ void __launch_bounds__(256) router_bwd_kernel(const uint16_t* __restr
   constexpr int KROW = KP + 4;  // padded LDS row of a dl tile (bf16)
   __shared__ __align__(16) uint16_t zt[4][32][kZRow];
   __shared__ __align__(16) uint16_t dt[4][32][KROW];
-  __shared__ float red[4][KP][65];
+  // above 32 routes (two workgroups of a CU then fit its LDS) the waves' tiles are
+  // added one after another, as router_dr_kernel adds them, over the dl tiles
+  constexpr int NR = KC <= 2 ? 4 : 1;
+  __shared__ float red_own[NR == 4 ? 4 : 1][NR == 4 ? KP : 1][65];
+  static_assert(NR == 4 || sizeof(float) * KP * 65 <= sizeof(dt), "the sums fit the dl tiles");
+  float(*red)[KP][65] = reinterpret_cast<float(*)[KP][65]>(NR == 4 ? static_cast<void*>(red_own) : dt);
   const int lane = threadIdx.x & 63, w = wave_id();
   const int i = lane & 15, qq = lane >> 4;
   const int zs = blockIdx.x * 64;
@@ -497,8 +510,18 @@ __global__ void __launch_bounds__(256) router_bwd_kernel(const uint16_t* __restr
   for (int tl = 0; tl < 4; ++tl)
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) acc[tl][kc] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // dz A operands: router[16 kc + 4 qq + v][zs + dz_col(tl, i)] (routes >= K load 0)
+  // dz A operands: router[16 kc + 4 qq + v][zs + dz_col(tl, i)] (routes >= K load
+  // 0); above 32 routes their 4 KC register pairs do not fit beside the
+  // accumulators, and they are read transposed from a tile of the router's columns
+  constexpr bool kALds = KC > 2;
+  __shared__ __align__(16) uint16_t rt[kALds ? KP : 1][kALds ? kZRow : 8];
   s16x4 aop[4][KC];
+  if constexpr (kALds) {
+    for (int c = threadIdx.x; c < KP * 8; c += 256)
+      *reinterpret_cast<u32x4*>(&rt[c / 8][8 * (c % 8)]) =
+          load16(rb, static_cast<uint32_t>(((c / 8) * Z + zs + 8 * (c % 8)) * 2));
+    __syncthreads();
+  } else {
 #pragma unroll
   for (int tl = 0; tl < 4; ++tl)
 #pragma unroll
@@ -513,6 +536,7 @@ __global__ void __launch_bounds__(256) router_bwd_kernel(const uint16_t* __restr
       aop[tl][kc] = s16x4{static_cast<short>(e[0]), static_cast<short>(e[1]),
                           static_cast<short>(e[2]), static_cast<short>(e[3])};
     }
+  }
 
   const int64_t blk0 = static_cast<int64_t>(blockIdx.y) * blocks_per_range;
   struct Regs {
@@ -557,27 +581,54 @@ __global__ void __launch_bounds__(256) router_bwd_kernel(const uint16_t* __restr
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc) ad[kc][h] = tr_read(&dt[w][row][16 * kc + 4 * a]);
     }
-    // dz B operands: dl[t0 + 16 hb + i][16 kc + 4 qq + {0..3}]
+    // dz B operands: dl[t0 + 16 hb + i][16 kc + 4 qq + {0..3}] (above 32 routes
+    // after the drouter products, whose operands' registers they take)
+    auto load_bd = [&]() {
 #pragma unroll
-    for (int hb = 0; hb < 2; ++hb)
+      for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
-      for (int kc = 0; kc < KC; ++kc)
-        bd[hb][kc] = *reinterpret_cast<const s16x4*>(&dt[w][16 * hb + i][16 * kc + 4 * qq]);
+        for (int kc = 0; kc < KC; ++kc)
+          bd[hb][kc] = *reinterpret_cast<const s16x4*>(&dt[w][16 * hb + i][16 * kc + 4 * qq]);
+    };
+    if constexpr (!kALds) load_bd();
 #pragma unroll
     for (int tl = 0; tl < 4; ++tl)
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc)
         acc[tl][kc] = mfma::mma32(ad[kc][0], ad[kc][1], bz[tl][0], bz[tl][1], acc[tl][kc]);
+    if constexpr (kALds) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_bd();
+    }
     const int64_t t0 = (blk0 + bb) * 32;
 #pragma unroll
-    for (int hb = 0; hb < 2; ++hb) {
-      f32x4 o[4];
+    for (int half = 0; half < 2; ++half) {
+      f32x4 o[2][2];
 #pragma unroll
-      for (int tl = 0; tl < 4; ++tl) o[tl] = dz_tile<KC>(aop[tl], bd[hb]);
-      const int64_t t = t0 + 16 * hb + i;
+      for (int th = 0; th < 2; ++th) {
+        const int tl = 2 * half + th;
+        if constexpr (kALds) {  // (dz_tile's chunk pairs, for both token blocks)
+          o[0][th] = o[1][th] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const f32x4 a0 = o[2 * half], a1 = o[2 * half + 1];
+          for (int kc = 0; kc < KC; kc += 2) {
+            const s16x4 zero = {0, 0, 0, 0};
+            const bool two = kc + 1 < KC;
+            const int col = 32 * half + 8 * a + 4 * th, k2 = two ? kc + 1 : kc;
+            const s16x4 a0 = tr_read(&rt[16 * kc + 4 * qq + e][col]);
+            const s16x4 a1 = two ? tr_read(&rt[16 * k2 + 4 * qq + e][col]) : zero;
+#pragma unroll
+            for (int hb = 0; hb < 2; ++hb)
+              o[hb][th] = mfma::mma32(a0, a1, bd[hb][kc], two ? bd[hb][k2] : zero, o[hb][th]);
+          }
+        } else {
+#pragma unroll
+          for (int hb = 0; hb < 2; ++hb) o[hb][th] = dz_tile<KC>(aop[tl], bd[hb]);
+        }
+      }
+#pragma unroll
+      for (int hb = 0; hb < 2; ++hb) {
+        const int64_t t = t0 + 16 * hb + i;
+        const f32x4 a0 = o[hb][0], a1 = o[hb][1];
         const u32x4 pk = {mfma::pack2_bf16(a0[0], a0[1]), mfma::pack2_bf16(a0[2], a0[3]),
                           mfma::pack2_bf16(a1[0], a1[1]), mfma::pack2_bf16(a1[2], a1[3])};
         const uint32_t off = static_cast<uint32_t>((t * Z + zs + 32 * half + 8 * qq) * 2);
@@ -591,32 +642,64 @@ __global__ void __launch_bounds__(256) router_bwd_kernel(const uint16_t* __restr
   // zero to two blocks left run after it, so the loop has a single exit and
   // the three sets stay in flight across its back edge.
   const int nb = (blocks_per_range - w + 3) / 4;
-  Regs r0, r1, r2;
+  Regs r0, r1;
   load_block(r0, w);
   load_block(r1, w + 4);
-  load_block(r2, w + 8);
   int it = 0;
-  for (; it + 3 <= nb; it += 3) {  // per wave; no barrier inside
-    const int b = w + 4 * it;
-    mult_block(r0, b);
-    load_block(r0, b + 12);
-    mult_block(r1, b + 4);
-    load_block(r1, b + 16);
-    mult_block(r2, b + 8);
-    load_block(r2, b + 20);
+  if constexpr (KC <= 2) {
+    Regs r2;
+    load_block(r2, w + 8);
+    for (; it + 3 <= nb; it += 3) {  // per wave; no barrier inside
+      const int b = w + 4 * it;
+      mult_block(r0, b);
+      load_block(r0, b + 12);
+      mult_block(r1, b + 4);
+      load_block(r1, b + 16);
+      mult_block(r2, b + 8);
+      load_block(r2, b + 20);
+    }
+    if (it < nb) mult_block(r0, w + 4 * it);
+    if (it + 1 < nb) mult_block(r1, w + 4 * it + 4);
+  } else {
+    for (; it + 2 <= nb; it += 2) {
+      const int b = w + 4 * it;
+      mult_block(r0, b);
+      load_block(r0, b + 8);
+      mult_block(r1, b + 4);
+      load_block(r1, b + 12);
+    }
+    if (it < nb) mult_block(r0, w + 4 * it);
   }
-  if (it < nb) mult_block(r0, w + 4 * it);
-  if (it + 1 < nb) mult_block(r1, w + 4 * it + 4);
+  if constexpr (NR == 4) {
 #pragma unroll
-  for (int tl = 0; tl < 4; ++tl)
+    for (int tl = 0; tl < 4; ++tl)
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc)
+      for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) red[w][16 * kc + 4 * qq + v][16 * tl + i] = acc[tl][kc][v];
-  __syncthreads();
+        for (int v = 0; v < 4; ++v) red[w][16 * kc + 4 * qq + v][16 * tl + i] = acc[tl][kc][v];
+    __syncthreads();
+  } else {
+    __syncthreads();  // every wave has read its dl tiles
+#pragma unroll
+    for (int ww = 0; ww < 4; ++ww) {
+      if (w == ww) {
+#pragma unroll
+        for (int tl = 0; tl < 4; ++tl)
+#pragma unroll
+          for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              float& cell = red[0][16 * kc + 4 * qq + v][16 * tl + i];
+              cell = ww == 0 ? acc[tl][kc][v] : cell + acc[tl][kc][v];
+            }
+      }
+      __syncthreads();
+    }
+  }
   for (int idx = threadIdx.x; idx < K * 64; idx += 256) {
     const int k = idx / 64, col = idx % 64;
-    const float sm = ((red[0][k][col] + red[1][k][col]) + red[2][k][col]) + red[3][k][col];
+    float sm = red[0][k][col];
+    if constexpr (NR == 4) sm = ((sm + red[NR - 3][k][col]) + red[NR - 2][k][col]) + red[NR - 1][k][col];
     part[(static_cast<int64_t>(blockIdx.y) * K + k) * Z + zs + col] = sm;
   }
 }
@@ -699,11 +782,24 @@ struct FwdLaunch {
   static void run(const uint16_t* z, const uint16_t* r, uint16_t* out, int64_t N, int Z, int K,
                   int routing, const RouteGroups& grp, hipStream_t st) {
     const dim3 grid(static_cast<unsigned>(cdiv(N, 32)));
+    if constexpr (KC > 2) {
+      // the four-block form where it gives every one of 256 CUs a workgroup
+      if (N >= 64 * 256) {
+        const dim3 grid4(static_cast<unsigned>(cdiv(N, 64)));
+        if (grp.n > 0)
+          hipLaunchKernelGGL((router_fwd_kernel<KC, true, 4>), grid4, dim3(256), 0, st, z, r, out, N, Z,
+                             K, routing, grp);
+        else
+          hipLaunchKernelGGL((router_fwd_kernel<KC, false, 4>), grid4, dim3(256), 0, st, z, r, out, N, Z,
+                             K, routing, grp);
+        return;
+      }
+    }
     if (grp.n > 0)
-      hipLaunchKernelGGL((router_fwd_kernel<KC, true>), grid, dim3(256), 0, st, z, r, out, N, Z, K,
+      hipLaunchKernelGGL((router_fwd_kernel<KC, true, 2>), grid, dim3(256), 0, st, z, r, out, N, Z, K,
                          routing, grp);
     else
-      hipLaunchKernelGGL((router_fwd_kernel<KC, false>), grid, dim3(256), 0, st, z, r, out, N, Z,
+      hipLaunchKernelGGL((router_fwd_kernel<KC, false, 2>), grid, dim3(256), 0, st, z, r, out, N, Z,
                          K, routing, grp);
   }
 };
@@ -724,6 +820,16 @@ struct DrLaunch {
                   const BwdPlan& pl, hipStream_t st) {
     const dim3 grid(static_cast<unsigned>(Z / 64), static_cast<unsigned>(pl.ranges));
     hipLaunchKernelGGL(router_dr_kernel<KC>, grid, dim3(256), 0, st, dl, z, part, N, Z, K,
+                       static_cast<int>(pl.blocks_per_range));
+  }
+};
+
+template <int KC>
+struct BwdLaunch {
+  static void run(const uint16_t* dl, const uint16_t* z, const uint16_t* r, uint16_t* dz, float* part,
+                  int64_t N, int Z, int K, const BwdPlan& pl, hipStream_t st) {
+    const dim3 grid(static_cast<unsigned>(Z / 64), static_cast<unsigned>(pl.ranges));
+    hipLaunchKernelGGL(router_bwd_kernel<KC>, grid, dim3(256), 0, st, dl, z, r, dz, part, N, Z, K,
                        static_cast<int>(pl.blocks_per_range));
   }
 };
@@ -766,16 +872,9 @@ void router_backward(const void* z, const void* r, const void* dl, void* dz, voi
   const int Zi = static_cast<int>(Z), Ki = static_cast<int>(K);
   const router::BwdPlan pl = router::bwd_plan(N, Z);
   float* part = static_cast<float*>(workspace);
-  // both outputs, K <= 32: one pass over z and dz
-  if (dz != nullptr && dr != nullptr && K <= 32) {
-    const dim3 grid(static_cast<unsigned>(Z / 64), static_cast<unsigned>(pl.ranges));
-    auto* op = static_cast<uint16_t*>(dz);
-    if (K <= 16)
-      hipLaunchKernelGGL(router::router_bwd_kernel<1>, grid, dim3(256), 0, st, dp, zp, rp, op,
-                         part, N, Zi, Ki, static_cast<int>(pl.blocks_per_range));
-    else
-      hipLaunchKernelGGL(router::router_bwd_kernel<2>, grid, dim3(256), 0, st, dp, zp, rp, op,
-                         part, N, Zi, Ki, static_cast<int>(pl.blocks_per_range));
+  // both outputs: one pass over z and dz
+  if (dz != nullptr && dr != nullptr) {
+    router::with_kc<router::BwdLaunch>(K, dp, zp, rp, static_cast<uint16_t*>(dz), part, N, Zi, Ki, pl, st);
     router::dr_reduce(part, dr, K, Z, pl, st);
     return;
   }

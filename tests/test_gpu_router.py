@@ -55,6 +55,24 @@ def test_router_forward_and_backward(N, Z, K):
     assert torch.equal(dr_only, dr)
 
 
+@pytest.mark.parametrize("N,Z,Ks", [(16383, 64, (32, 4)), (16384, 128, (16, 32)), (16385, 192, (32, 32)),
+                                    (16400, 64, (32, 32, 12)), (16447, 320, (32, 32, 32))])
+def test_router_many_routes_many_tokens(N, Z, Ks):
+    """33 to 96 routes around the token count from which a forward workgroup
+    takes 64 tokens, single and grouped, and the one-pass backward."""
+    K = sum(Ks)
+    z, r, dl = _inputs(N, Z, K, N + Z + K)
+    logits = ops.router_forward(z, r)
+    assert_close("logits", logits, z.float() @ r.float().T, BF)
+    parts = r.split(Ks)
+    ws = ops.router_forward_grouped(z, r, list(Ks), [ops.ROUTE_ALPHA] * len(Ks))
+    for w, p in zip(ws, parts):
+        assert torch.equal(w, ops.router_forward(z, p.contiguous()))
+    dz, dr = ops.router_backward(z, r, dl, True, True)
+    assert_close("dz", dz, dl.float() @ r.float(), BF)
+    assert_close("drouter", dr, dl.float().T @ z.float(), BF)
+
+
 def test_router_batched_input_and_autograd():
     B, T, Z, K = 3, 37, 128, 16
     g = gen(5)
