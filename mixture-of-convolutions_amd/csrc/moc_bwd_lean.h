@@ -1,4 +1,5 @@
-// Fused backward (stage 1) with 2 to 8 taps: bf16 up to 32 routes, fp32 up to 16.
+// Fused backward (stage 1) with 2 to 8 taps: bf16 up to 32 routes, fp32 up to 16
+// (32 with up to 5 taps).
 //
 // What bounds it: instruction issue and the latency chains of two to four waves
 // per SIMD (four, 128 VGPRs, with 2 to 4 taps and 16 routes; else two, 256 VGPRs).
@@ -38,7 +39,13 @@
 //         111->(114)   170->132     206->158     249->184     260->209     330->263
 //         132->118     180->137     273->165     342->193     352->223     484->282
 // B4 T2048 D1024, 4 taps, SiLU: 92 -> 54, its training step 145 -> 108; same
-// order at 4 routes, D 4096, and 600 rows of D 3000.
+// order at 4 routes, D 4096, and 600 rows of D 3000.  32 routes, to 5 taps (six
+// taps' basis tiles are past a CU's LDS), the fused pass (2, 3 taps) or the two
+// passes -> here:
+//   taps  2            3            4            5
+//         226->204     287->237     322->268     424->318
+//         253->185     356->228     414->276     546->320
+// B4 T2048 D1024, 4 taps, SiLU: 129 -> 85.
 //
 // Work per step and wave (rows 8 i .. 8 i + 7 of each stream):
 //   W_s = alpha . basis_s by MFMA (16x16x16, or 16x16x32 over 32 routes; both
@@ -89,7 +96,7 @@ constexpr int kLeanCW = 16;        // channels per wave
 // Shapes the lean pass serves (fp32 with 2 taps and no activation, where there is
 // little to form or share: 111 us in the fused pass of bwd_tile, 114 here)
 constexpr bool bwd_lean(int S, int KC, bool act, bool bf) {
-  return KC <= (bf ? 2 : 1) && S >= 2 && S <= 8 && (bf || act || S > 2);
+  return S >= 2 && (bf ? KC <= 2 && S <= 8 : (KC == 1 && S <= 8 && (act || S > 2)) || (KC == 2 && S <= 5));
 }
 // Waves per SIMD it is built for: four (128 VGPRs, two workgroups per CU) with 2
 // to 4 taps and 16 routes in bf16, else two (256 VGPRs and up to 156 KB of LDS,
@@ -145,7 +152,6 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
   constexpr int KP = 16 * KC, WPG = kLeanWPG, CW = kLeanCW;
   constexpr int ESZ = sizeof(E);
   static_assert(S >= 2 && S <= 8 && KC <= 2, "lean backward: 2 to 8 taps, up to 32 routes");
-  static_assert(BF || KC == 1, "fp32: up to 16 routes");
   // the four-wave form leaves what a stream owes its predecessor in LDS
   constexpr bool kC0Lds = lean_waves(S, KC, BF) == 4;
   // The next step's rows are loaded where this step's have been converted in the
@@ -161,13 +167,16 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
   auto asw = [](int row) -> int {
     return KC == 1 ? (row >> 3) & 3 : ((row >> 1) & 1) | (((row >> 3) & 3) << 1);
   };
-  __shared__ __align__(16) E a_lds[2][BF ? TB : 1][BF ? KP : kF32Rows];
+  __shared__ __align__(16) E a_lds[2][BF ? TB : KC][BF ? KP : kF32Rows];
   __shared__ __align__(16) Op m_tr[BF ? WPG : 1][2][TrTile1::kSlots];  // [wave][hi / lo]
   __shared__ __align__(16) float m_f32[BF ? 1 : WPG][kF32Rows];        // fp32: rows x channels
   // basis tile of each wave, b_lds[wave][s][kc][route j][4 channels, chunk q ^
   // (j / 4)] (a 16-lane group of a read touches 16 distinct slots)
   __shared__ __align__(16) Op b_lds[WPG][S][KC][BF ? 16 * 4 : kF32Basis / 4];
-  __shared__ float da_lds[2][WPG][NB][KC][16][17];
+  // (fp32 over 32 routes: one buffer, the two of them past the CU's LDS, and a
+  // second barrier in a step)
+  constexpr int DAB = BF || KC == 1 ? 2 : 1;
+  __shared__ float da_lds[DAB][WPG][NB][KC][16][17];
   __shared__ float c0_lds[kC0Lds ? H : 1][kC0Lds ? 64 * WPG : 1];
 
   const int tid = threadIdx.x;
@@ -286,7 +295,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
     if (wave < 2 * KC) {
       const int t = opaque_tid(), row = t / (4 * KC);
       if constexpr (BF) Vec<E, 4>::store(&a_lds[buf][row][((t % (4 * KC)) ^ asw(row)) * 4], arw);
-      else Vec<E, 4>::store(&a_lds[buf][0][f32_aslot(row, t % 4)], arw);
+      else Vec<E, 4>::store(&a_lds[buf][KC == 1 ? 0 : t % (4 * KC) / 4][f32_aslot(row, t % 4)], arw);
     }
   };
 
@@ -360,7 +369,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
         if constexpr (BF)
           aop[b][kc] = *reinterpret_cast<const Op*>(&a_lds[buf][row][((4 * kc + q) ^ asw(row)) * 4]);
         else
-          aop[b][kc] = *reinterpret_cast<const Op*>(&a_lds[buf][0][f32_aslot(row, q)]);
+          aop[b][kc] = *reinterpret_cast<const Op*>(&a_lds[buf][kc][f32_aslot(row, q)]);
       }
 
     f32x4 dacc[NB][KC];
@@ -416,7 +425,8 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
           const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-          if constexpr (KC == 2) w[b] = mma32(aop[b][0], aop[b][1], bop[0], bop[1], zero);
+          if constexpr (KC == 2 && !BF) w[b] = C::mma(aop[b][1], bop[1], C::mma(aop[b][0], bop[0], zero));
+          else if constexpr (KC == 2) w[b] = mma32(aop[b][0], aop[b][1], bop[0], bop[1], zero);
           else w[b] = C::mma(aop[b][0], bop[0], zero);
         }
       };
@@ -491,7 +501,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
           } else {
 #pragma unroll
             for (int v = 0; v < 4; ++v)
-              at[b][kc][v] = a_lds[buf][0][f32_aslot(R * q + 4 * b + v, j >> 2) + (j & 3)];
+              at[b][kc][v] = a_lds[buf][kc][f32_aslot(R * q + 4 * b + v, j >> 2) + (j & 3)];
           }
         }
       if (!more) {
@@ -506,8 +516,10 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
               at[b][kc] = __builtin_bit_cast(Op, __builtin_bit_cast(uint64_t, at[b][kc]) & keep);
           } else {
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-              if (q == 3 && v >= n_ok) at[b][0][v] = 0.f;
+            for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+              for (int v = 0; v < 4; ++v)
+                if (q == 3 && v >= n_ok) at[b][kc][v] = 0.f;
           }
         }
       }
@@ -570,10 +582,13 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
           for (int r = 0; r < R; ++r) {
             const float mval = tap_ok(r, s) ? g[r] * xw[r + s] : 0.f;
             m_f32[wave][f32_mslot(R * q + r, j >> 2) + (j & 3)] = mval;
-            dbacc[s][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(mval, at[r >> 2][0][r & 3], dbacc[s][0], 0, 0, 0);
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc)
+              dbacc[s][kc] =
+                  __builtin_amdgcn_mfma_f32_16x16x4f32(mval, at[r >> 2][kc][r & 3], dbacc[s][kc], 0, 0, 0);
           }
         };
-        Op ra[NB], bda;
+        Op ra[NB], bda[KC];
         stage_m(0);
 #pragma unroll
         for (int s = 0; s < S; ++s) {
@@ -581,11 +596,14 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
 #pragma unroll
           for (int r2 = 0; r2 < NB; ++r2)
             ra[r2] = *reinterpret_cast<const Op*>(&m_f32[wave][f32_mslot(16 * r2 + j, q)]);
-          bda = b_lds[wave][s][0][f32_bslot(j, q) / 4];
+#pragma unroll
+          for (int kc = 0; kc < KC; ++kc) bda[kc] = b_lds[wave][s][kc][f32_bslot(j, q) / 4];
           __builtin_amdgcn_sched_barrier(0);
           if (s + 1 < S) stage_m(s + 1);
 #pragma unroll
-          for (int r2 = 0; r2 < NB; ++r2) dacc[r2][0] = C::mma(ra[r2], bda, dacc[r2][0]);
+          for (int r2 = 0; r2 < NB; ++r2)
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc) dacc[r2][kc] = C::mma(ra[r2], bda[kc], dacc[r2][kc]);
         }
       }
       wave_lds_sync();
@@ -599,7 +617,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) da_lds[buf][wave][r2][kc][4 * q + v][j] = dacc[r2][kc][v];
+        for (int v = 0; v < 4; ++v) da_lds[buf % DAB][wave][r2][kc][4 * q + v][j] = dacc[r2][kc][v];
     if (more) stage_alpha(buf ^ 1);
     __syncthreads();
     // sum the 8 waves' dalpha tiles in wave order; rows past the own ones drop
@@ -611,7 +629,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
-        for (int w = 0; w < WPG; ++w) tv[kc][w] = da_lds[buf][w][r2][kc][row][c];
+        for (int w = 0; w < WPG; ++w) tv[kc][w] = da_lds[buf % DAB][w][r2][kc][row][c];
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc) {
         float sum = 0.f;
@@ -619,6 +637,7 @@ bwd_lean_tile(const void* __restrict__ xv, const void* __restrict__ dyv, int64_t
         for (int w = 0; w < WPG; ++w) sum += tv[kc][w];
         pdb.store<4>(off + 64 * kc, &sum);
       }
+      if constexpr (DAB == 1) __syncthreads();
     }
   };
   // plain steps in a loop of their own: the accumulators stay in their registers

@@ -18,7 +18,7 @@ namespace mfma {
 #define MOC_FWD_NC 2
 #endif
 // 8 taps with one token block per super-block (11 window rows instead of 15,
-// 135 VGPRs, three waves per SIMD) measured slower at configs[4]: 1237 -> 1251 us
+// 135 VGPRs, three waves per SIMD) measured slower on the QKV step of 4096 / 1024 / 1024 channels: 1237 -> 1251 us
 #ifndef MOC_FWD_NB8
 #define MOC_FWD_NB8 2
 #endif
@@ -181,18 +181,16 @@ inline Grid2 bwd_grid_tiered(int64_t N, int64_t gx, int64_t D, int64_t S, int n_
 // against the fused pass at every kernel size: below those the fused pass is
 // faster), and 9 to 16 taps.
 // fp32 (the same two passes on fp32 operands, with and without the activation):
-// 16 routes from 5 taps (4 without the activation) to 16, 32 routes from 4 to
-// 8 taps.  Past 8 taps the fused fp32 tile does not build (its register file);
-// below, measured against the fused pass (B4 T4096 D2048, backward entry, us,
-// without / with SiLU): 16 routes, 4 taps 234 / 290 -> 222 / 295, 6 taps
-// 323 / 414 -> 275 / 356, 8 taps 463 / 562 -> 354 / 461; 32 routes, 4 taps
-// 381 / 464 -> 324 / 415, 6 taps 1177 / 1427 -> 450 / 615, 8 taps
+// 16 routes past 8 taps, where the fused fp32 tile does not build (its register
+// file), and 32 routes with 6 to 8 taps, whose basis tiles the lean pass's LDS
+// does not hold; against the fused pass (B4 T4096 D2048, backward entry, us,
+// without / with SiLU): 32 routes, 6 taps 1177 / 1427 -> 450 / 615, 8 taps
 // 1046 / 1425 -> 704 / 986.
-constexpr bool f32_two_pass(int S, int KC, bool act) {
-  return (KC == 1 && (S >= 5 || (S == 4 && !act))) || (KC == 2 && S >= 4 && S <= 8);
+constexpr bool f32_two_pass(int S, int KC) {
+  return (KC == 1 && S > 8) || (KC == 2 && S >= 6 && S <= 8);
 }
 constexpr bool bwd_two_pass(int S, int KC, bool act, bool bf) {
-  return !act && ((bf && ((KC == 2 && S >= 4) || (KC == 1 && S >= 7))) || (!bf && f32_two_pass(S, KC, act)));
+  return !act && ((bf && ((KC == 2 && S >= 4) || (KC == 1 && S >= 7))) || (!bf && f32_two_pass(S, KC)));
 }
 // With the activation, the two passes where the fused pass spills or forms the
 // same work per route chunk (bf16: 64 routes and 3 to 8 taps, 9 to 16 taps, and
@@ -201,7 +199,7 @@ constexpr bool bwd_two_pass(int S, int KC, bool act, bool bf) {
 // taps pass.  Single launches only (the grouped launch keeps the fused pass).
 constexpr bool bwd_two_pass_g(int S, int KC, bool act, bool bf) {
   return act && ((bf && ((KC == 2 && S >= 5) || (KC == 1 && S >= 8) || (KC == 4 && S >= 3))) ||
-                 (!bf && f32_two_pass(S, KC, act)));
+                 (!bf && f32_two_pass(S, KC)));
 }
 // The prefill runs those two passes (the dx pass's P reading the cache) with 32
 // routes and 6-8 taps and with 64 routes; elsewhere its fused pass measured

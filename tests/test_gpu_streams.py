@@ -1,5 +1,5 @@
 """The stream form of the fused backward (2 to 8 taps; bf16 up to 32 routes, fp32
-up to 16):
+up to 16, and 32 with up to 5 taps):
 ranges of one and of several steps, token counts around a step and a range, a
 ragged last channel group, segment starts at every place of a stream (between
 streams, steps and ranges included), against the oracle."""
@@ -76,7 +76,8 @@ def test_stream_broadcast_dy(form, S, K):
 
 @pytest.mark.parametrize("S,K,act", [(2, 16, "silu"), (3, 7, None), (4, 16, "silu"), (4, 4, None),
                                      (5, 12, None), (6, 16, "silu"), (7, 9, "silu"), (8, 16, "silu"),
-                                     (8, 16, None)])
+                                     (8, 16, None), (2, 32, "silu"), (3, 20, None), (4, 32, "silu"),
+                                     (5, 24, None), (5, 32, "silu")])
 @pytest.mark.parametrize("B,T,D", [(1, 1, 2), (1, 28, 16), (1, 29, 18), (1, 32, 128), (2, 33, 130),
                                    (1, 64, 254), (3, 5, 66)])
 def test_stream_edges_fixed_f32(S, K, act, B, T, D):
@@ -85,7 +86,8 @@ def test_stream_edges_fixed_f32(S, K, act, B, T, D):
            randn(g, K, S, D, scale=0.3), randn(g, B, T, D), act, dt=F32)
 
 
-@pytest.mark.parametrize("S,K,act", [(2, 12, None), (4, 16, "silu"), (4, 12, None), (8, 16, "silu")])
+@pytest.mark.parametrize("S,K,act", [(2, 12, None), (4, 16, "silu"), (4, 12, None), (8, 16, "silu"),
+                                     (4, 32, "silu"), (5, 20, None)])
 @pytest.mark.parametrize("longest", [3, 700])
 def test_stream_ranges_packed_f32(S, K, act, longest):
     # 128 ranges of the two channel groups, two to four steps each
@@ -101,7 +103,7 @@ def test_stream_ranges_packed_f32(S, K, act, longest):
 
 
 @pytest.mark.parametrize("form", ["one", "row"])
-@pytest.mark.parametrize("S,K,act", [(4, 16, "silu"), (8, 7, None)])
+@pytest.mark.parametrize("S,K,act", [(4, 16, "silu"), (8, 7, None), (4, 32, None)])
 def test_stream_broadcast_dy_f32(form, S, K, act):
     g = gen(7)
     B, T, D = 1, 128 * 29 + 1, 258
