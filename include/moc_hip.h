@@ -374,7 +374,8 @@ int moc_router_backward(const void* z, const void* router, const void* dlogits, 
  * after it (moc/api.py:383-388) and its backward on fp32 tensors: out = the
  * logits (routing 0), softmax_k (1) or exp (2) of them, [n_tokens, k].  Sums are
  * fp32, drouter's in a fixed order.  k % 4 == 0, k <= 32, z_dim % 64 == 0,
- * n_tokens * z_dim < 2^29 (moc_router_f32_supported returns 1 for such shapes).
+ * n_tokens * z_dim < 2^29 and z_dim times k rounded up to 16 or 32 < 2^29
+ * (moc_router_f32_supported returns 1 for such shapes).
  * dz or drouter may be NULL.
  */
 int moc_router_f32_supported(int64_t n_tokens, int64_t z_dim, int64_t k);

@@ -815,7 +815,8 @@ int moc_router_f32_supported(int64_t n_tokens, int64_t z_dim, int64_t k) {
 static int check_router_f32(int64_t n_tokens, int64_t z_dim, int64_t k) {
   if (moc::router_f32_supported(n_tokens, z_dim, k)) return 0;
   return fail(MOC_ERR_ARG, "fp32 router shape not supported (n_tokens %lld, z_dim %lld, k %lld): "
-                           "k %% 4 == 0, k <= %d, z_dim %% 64 == 0, n_tokens z_dim < 2^29",
+                           "k %% 4 == 0, k <= %d, z_dim %% 64 == 0, n_tokens z_dim and k z_dim "
+                           "(k in 16s) < 2^29",
               (long long)n_tokens, (long long)z_dim, (long long)k, moc::kRouterMaxRoutedK);
 }
 

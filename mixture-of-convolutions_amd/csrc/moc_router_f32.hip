@@ -177,7 +177,7 @@ router_f32_bwd_kernel(const float* __restrict__ dl, const float* __restrict__ z,
     const int t = 16 * blk;  // (blocks past the range lie past the buffers)
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      g.z[s] = load4(zb, static_cast<uint32_t>(((t + 4 * s + q) * Z + zs + 4 * i) * 4));
+      g.z[s] = load4(zb, (static_cast<uint32_t>(t + 4 * s + q) * static_cast<uint32_t>(Z) + zs + 4 * i) * 4);
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) {
       g.b[kc] = load4(db, 16 * kc + 4 * q < K ? static_cast<uint32_t>(((t + i) * K + 16 * kc + 4 * q) * 4) : kOffNone);
@@ -194,7 +194,7 @@ router_f32_bwd_kernel(const float* __restrict__ dl, const float* __restrict__ z,
         f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kc = 0; kc < KC; ++kc) o = mma4(aop[tl][kc], g.b[kc], o);
-        ob.store<16>(static_cast<uint32_t>(((16 * blk + i) * Z + zs + 16 * tl + 4 * q) * 4), &o);
+        ob.store<16>((static_cast<uint32_t>(16 * blk + i) * static_cast<uint32_t>(Z) + zs + 16 * tl + 4 * q) * 4, &o);
       }
     }
     if (part != nullptr) {
@@ -268,9 +268,13 @@ F32Plan f32_plan(int64_t N, int64_t Z) {
 }  // namespace
 }  // namespace router
 
+// The kernels address z and the router with 32-bit byte offsets: n_tokens z_dim and
+// the router with its routes padded to a tile (16 or 32 rows, also the 16 token
+// rows of a block past the last one) are below 2^29 elements each.
 bool router_f32_supported(int64_t N, int64_t Z, int64_t K) {
+  const int64_t lim = int64_t(1) << 29;
   return K > 0 && K <= kRouterMaxRoutedK && K % 4 == 0 && Z >= 64 && Z % 64 == 0 && N > 0 &&
-         N <= (int64_t(1) << 30) && N * Z < (int64_t(1) << 29);
+         N <= (int64_t(1) << 30) && Z < lim / 16 && N * Z < lim && router::cdiv(K, 16) * 16 * Z < lim;
 }
 
 void router_f32_forward(const void* z, const void* r, void* out, int64_t N, int64_t Z, int64_t K,

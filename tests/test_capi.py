@@ -118,6 +118,28 @@ def test_dtype_codes():
     assert isinstance(_lib.lib(), ctypes.CDLL)
 
 
+@pytest.mark.parametrize("n,z,k,ok", [
+    (4, (1 << 24) - 64, 32, 1), (4, 1 << 24, 32, 0),    # 32 rows of the router: 2^29 elements
+    (4, (1 << 25) - 64, 16, 1), (4, 1 << 25, 16, 0),
+    (4, (1 << 25) - 64, 4, 1), (1, 1 << 25, 4, 0),      # k is padded to 16 rows, a token block has 16
+    (4, 1 << 24, 20, 0), (15, 1 << 25, 32, 0),
+    ((1 << 23) - 1, 64, 4, 1), (1 << 23, 64, 4, 0),     # z itself
+])
+def test_router_f32_takes_what_32_bit_offsets_reach(n, z, k, ok):
+    """fp32 z and router are addressed with 32-bit byte offsets: shapes past them
+    are refused (the layer then takes torch's router), and the entries with them."""
+    L = _lib.lib()
+    assert L.moc_router_f32_supported(n, z, k) == ok
+    if ok:
+        # the largest offset a block may form, in bytes: its last row, past N or not
+        assert 4 * (n + 15) * z < 1 << 32 and (k + 15) // 16 * 16 * z * 4 < 1 << 31
+        assert L.moc_router_f32_backward_workspace_bytes(n, z, k) > 0
+    else:
+        assert L.moc_router_f32_backward_workspace_bytes(n, z, k) == 0
+        assert L.moc_router_f32_forward(FAKE, FAKE, FAKE, n, z, k, 0, None) == ERR_ARG
+        assert L.moc_router_f32_backward(FAKE, FAKE, FAKE, FAKE, None, n, z, k, None, 0, None) == ERR_ARG
+
+
 def test_router_grouped_rejects_bad_groups():
     """moc_router_forward_grouped validates its group arrays before any launch."""
     L = _lib.lib()
