@@ -751,10 +751,13 @@ BwdPlan bwd_plan(int64_t N, int64_t Z) {
 }  // namespace router
 
 bool router_supported(int64_t N, int64_t Z, int64_t K, int dt) {
-  // buffer resources address [N, Z] bf16 with 32-bit byte offsets; the dz grid
-  // (N / 64 token blocks at most) stays within the 65535 limit of grid.y
+  // buffer resources address [N, Z] and [K, Z] bf16 (K padded to 16s, token blocks
+  // of 32 rows) with 32-bit byte offsets; the dz grid (N / 64 token blocks at most)
+  // stays within the 65535 limit of grid.y
+  const int64_t lim = int64_t(1) << 30;
   return dt == DT_BF16 && K > 0 && K <= kRouterMaxK && K % 4 == 0 && Z >= 64 && Z % 64 == 0 &&
-         N > 0 && N * Z * 2 < (int64_t(1) << 31) && N <= int64_t(65535) * 64;
+         N > 0 && Z < lim / 32 && N * Z < lim && router::cdiv(K, 16) * 16 * Z < lim &&
+         N <= int64_t(65535) * 64;
 }
 
 size_t router_backward_workspace(int64_t N, int64_t Z, int64_t K) {

@@ -140,6 +140,22 @@ def test_router_f32_takes_what_32_bit_offsets_reach(n, z, k, ok):
         assert L.moc_router_f32_backward(FAKE, FAKE, FAKE, FAKE, None, n, z, k, None, 0, None) == ERR_ARG
 
 
+@pytest.mark.parametrize("n,z,k,ok", [
+    (4, (1 << 25) - 64, 32, 1), (4, 1 << 25, 32, 0), (1, 1 << 25, 4, 0),
+    (8, (1 << 30) // 96 // 64 * 64, 96, 1), (8, (1 << 30) // 96 // 64 * 64 + 64, 96, 0),
+    (4, 1 << 24, 52, 0), (16384, 65536 - 64, 96, 1), (16384, 65536, 96, 0),
+])
+def test_router_takes_what_32_bit_offsets_reach(n, z, k, ok):
+    """The same for the bf16 router (blocks of up to 64 token rows)."""
+    L = _lib.lib()
+    assert L.moc_router_supported(n, z, k, _lib.DT_BF16) == ok
+    if ok:
+        assert 2 * ((n + 63) // 64 * 64) * z < 1 << 32 and (k + 15) // 16 * 16 * z * 2 < 1 << 31
+    else:
+        assert L.moc_router_forward(FAKE, FAKE, FAKE, n, z, k, _lib.DT_BF16, None) == ERR_ARG
+        assert L.moc_router_backward_workspace_bytes(n, z, k, _lib.DT_BF16) == 0
+
+
 def test_router_grouped_rejects_bad_groups():
     """moc_router_forward_grouped validates its group arrays before any launch."""
     L = _lib.lib()
