@@ -30,7 +30,7 @@ using OptTensor = std::optional<Tensor>;
 
 int dtype_code(at::ScalarType t) { return t == at::kFloat ? 0 : (t == at::kBFloat16 ? 1 : -1); }
 
-// A dense GPU tensor of its own: no subclass or transform of one, no dual number.
+// A dense GPU tensor of its own: no wrapper or transform of one, no dual number.
 bool plain(const Tensor& t) {
   if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.is_neg() || t.is_conj()) return false;
   static const c10::DispatchKeySet wrapped({DispatchKey::Python, DispatchKey::PythonTLSSnapshot,
@@ -360,12 +360,45 @@ void name_node(const char* name) {
   torch::autograd::registerCppFunction(typeid(torch::autograd::CppNode<F>), &type);
 }
 
+// A call's tensor arguments as Python hands them over.  Only torch.Tensor and
+// torch.nn.Parameter themselves are taken: a subclass, with or without a dispatch
+// key of its own, keeps its result type and its __torch_function__ in the Python
+// functions, and what is no tensor its error there.
+struct Args {
+  bool own = true;
+  Tensor operator()(py::handle h) {
+    own = own && THPVariable_CheckExact(h.ptr());
+    return own ? THPVariable_Unpack(h.ptr()) : Tensor();
+  }
+  OptTensor opt(py::handle h) { return h.is_none() ? OptTensor() : OptTensor((*this)(h)); }
+};
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   name_node<LayerFn>("_MoCLayerFunctionBackward");
   name_node<FuncFn>("_MoCFunctionBackward");
-  m.def("layer", &layer);
-  m.def("func", &func);
-  m.def("stateful", &stateful);
+  m.def("layer", [](py::handle x, py::handle z, py::handle router, py::handle basis, int act, int route,
+                    py::handle cu) -> OptTensor {
+    Args a;
+    const Tensor tx = a(x), tz = a(z), tr = a(router), tb = a(basis);
+    const OptTensor tc = a.opt(cu);
+    if (!a.own) return std::nullopt;
+    return layer(tx, tz, tr, tb, act, route, tc);
+  });
+  m.def("func", [](py::handle x, py::handle alpha, py::handle basis, int act, py::handle cu) -> OptTensor {
+    Args a;
+    const Tensor tx = a(x), ta = a(alpha), tb = a(basis);
+    const OptTensor tc = a.opt(cu);
+    if (!a.own) return std::nullopt;
+    return func(tx, ta, tb, act, tc);
+  });
+  m.def("stateful", [](py::handle x, py::handle z, py::handle router, py::handle basis, py::handle cache, int act,
+                       int route, bool want) -> std::optional<std::tuple<Tensor, OptTensor>> {
+    Args a;
+    const Tensor tx = a(x), tz = a(z), tr = a(router), tb = a(basis);
+    const OptTensor tc = a.opt(cache);
+    if (!a.own) return std::nullopt;
+    return stateful(tx, tz, tr, tb, tc, act, route, want);
+  });
 }

@@ -147,6 +147,33 @@ def test_watched_calls_stay_with_python():
     assert H.layer(x[:, :0], z[:, :0], *args) is None and H.layer(x, z[:, :5], *args) is None
 
 
+class Tagged(torch.Tensor):
+    """A subclass without __torch_dispatch__: nothing in its dispatch keys."""
+
+
+def test_subclasses_keep_their_type():
+    m, g = _layer(BF), gen(11)
+    x, z = randn(g, 2, 20, 130).to(DEV, BF), randn(g, 2, 20, 128).to(DEV, BF)
+    a = randn(g, 2, 20, 16).to(DEV, BF)
+    tx, H = x.as_subclass(Tagged), _lib.host()
+    assert H.layer(tx, z, m.router, m.conv_bases, 1, 1, None) is None
+    assert H.layer(x, z.as_subclass(Tagged), m.router, m.conv_bases, 1, 1, None) is None
+    assert H.func(x, a.as_subclass(Tagged), m.conv_bases, 1, None) is None
+    assert H.stateful(x, z, m.router.as_subclass(Tagged), m.conv_bases, None, 1, 1, True) is None
+    for grad in (True, False):
+        with torch.set_grad_enabled(grad):
+            for got, want in ((m(tx, z)[0], m(x, z)[0]),
+                              (moc.moc_triton(tx, a, m.conv_bases)[0], moc.moc_triton(x, a, m.conv_bases)[0])):
+                assert type(got) is Tagged and type(want) is torch.Tensor
+                assert torch.equal(got.as_subclass(torch.Tensor), want)
+    with torch.no_grad():
+        y, cache = m.step(tx[:, :1], z[:, :1], cache=torch.zeros(2, 130, 4, device=DEV, dtype=BF))
+        assert type(y) is Tagged
+    # what is no tensor gets the Python functions' error, not an argument error
+    with pytest.raises(AttributeError):
+        moc.moc_triton(x[0], a[0], m.conv_bases, cu_seqlens=[0, 20], max_seqlen=20)
+
+
 @pytest.mark.parametrize("dtype", [BF, F32])
 def test_stateful_bit_for_bit(dtype):
     m, g = _layer(dtype), gen(9)
