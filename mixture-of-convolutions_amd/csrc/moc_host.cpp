@@ -363,7 +363,10 @@ void name_node(const char* name) {
 // A call's tensor arguments as Python hands them over.  Only torch.Tensor and
 // torch.nn.Parameter themselves are taken: a subclass, with or without a dispatch
 // key of its own, keeps its result type and its __torch_function__ in the Python
-// functions, and what is no tensor its error there.
+// functions, and what is no tensor its error there.  The calls then run without the
+// interpreter lock: an allocation may wait for the device and a launch for space in
+// the queue, and other threads' work goes on meanwhile (saved-tensor hooks take the
+// lock themselves).
 struct Args {
   bool own = true;
   Tensor operator()(py::handle h) {
@@ -384,6 +387,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     const Tensor tx = a(x), tz = a(z), tr = a(router), tb = a(basis);
     const OptTensor tc = a.opt(cu);
     if (!a.own) return std::nullopt;
+    const py::gil_scoped_release unlocked;
     return layer(tx, tz, tr, tb, act, route, tc);
   });
   m.def("func", [](py::handle x, py::handle alpha, py::handle basis, int act, py::handle cu) -> OptTensor {
@@ -391,6 +395,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     const Tensor tx = a(x), ta = a(alpha), tb = a(basis);
     const OptTensor tc = a.opt(cu);
     if (!a.own) return std::nullopt;
+    const py::gil_scoped_release unlocked;
     return func(tx, ta, tb, act, tc);
   });
   m.def("stateful", [](py::handle x, py::handle z, py::handle router, py::handle basis, py::handle cache, int act,
@@ -399,6 +404,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     const Tensor tx = a(x), tz = a(z), tr = a(router), tb = a(basis);
     const OptTensor tc = a.opt(cache);
     if (!a.own) return std::nullopt;
+    const py::gil_scoped_release unlocked;
     return stateful(tx, tz, tr, tb, tc, act, route, want);
   });
 }

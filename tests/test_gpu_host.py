@@ -3,7 +3,9 @@ functions they stand for: bit for bit over the forms both take, and what autogra
 promises of a node kept: hooks on saved tensors, version checks, partial
 gradients, one differentiation; transforms, tracing and forward mode stay with
 the Python functions."""
+import sys
 import threading
+import time
 
 import pytest
 import torch
@@ -196,21 +198,71 @@ def test_stateful_bit_for_bit(dtype):
         assert (y - ref).float().abs().max() <= 2.0 ** -7 * ref.float().abs().max()
 
 
-def test_streams_and_threads():
-    m, g = _layer(BF), gen(10)
-    sets = [(randn(g, 2, 300, 130).to(DEV, BF), randn(g, 2, 300, 128).to(DEV, BF)) for _ in range(4)]
-    want = [m(x, z)[0].detach().clone() for x, z in sets]
+def _step(m, x, z, dy):
+    y, _ = m(x, z)
+    return [y.detach(), *torch.autograd.grad(y, [x, z, m.router, m.conv_bases], dy)]
+
+
+@pytest.mark.parametrize("dtype", [BF, F32])
+def test_streams_and_threads(dtype):
+    """Forward and backward of four threads at once, each on a stream of its own."""
+    m, g = _layer(dtype), gen(10)
+    sets = [tuple(randn(g, 2, 300, n).to(DEV, dtype) for n in (130, 128, 130)) for _ in range(4)]
+    sets = [(x.requires_grad_(), z.requires_grad_(), dy) for x, z, dy in sets]
+    want = [_step(m, *s) for s in sets]
     torch.cuda.synchronize()
     got = [None] * 4
+    together = threading.Barrier(4)
 
     def work(i):
         s = torch.cuda.Stream()
         with torch.cuda.stream(s):
+            together.wait()
             for _ in range(20):
-                got[i] = m(*sets[i])[0].detach()
+                got[i] = _step(m, *sets[i])
         s.synchronize()
 
     threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
     [t.start() for t in threads]
     [t.join() for t in threads]
-    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert all(torch.equal(u, v) for a, b in zip(got, want) for u, v in zip(a, b))
+
+
+def test_other_threads_run_during_a_call():
+    """The calls run without the interpreter lock: with no switch forced (an
+    interval of 100 s), another thread counts on only while a call is inside."""
+    m, g = _layer(BF), gen(12)
+    x, z = randn(g, 2, 2000, 130).to(DEV, BF), randn(g, 2, 2000, 128).to(DEV, BF)
+    w = randn(g, 2, 2000, 16).to(DEV, BF)
+    c0 = randn(g, 2, 130, 4).to(DEV, BF)
+    H = _lib.host()
+    calls = {"layer": lambda: H.layer(x, z, m.router, m.conv_bases, 1, 1, None),
+             "func": lambda: H.func(x, w, m.conv_bases, 1, None),
+             "stateful": lambda: H.stateful(x, z, m.router, m.conv_bases, c0, 1, 1, True)}
+    count, stop = [0], []
+
+    def other():
+        while not stop:
+            count[0] += 1
+            time.sleep(0)  # gives the lock up and waits for it again
+
+    before = sys.getswitchinterval()
+    thread = threading.Thread(target=other)
+    try:
+        sys.setswitchinterval(100.0)
+        thread.start()
+        for name, call in calls.items():
+            ran = 0
+            for _ in range(30):
+                torch.cuda.empty_cache()  # the call allocates from the device: long enough to switch
+                at = count[0]
+                with torch.set_grad_enabled(name != "stateful"):
+                    out = call()
+                ran += count[0] - at
+                assert out is not None
+                del out
+            assert ran > 0, name
+    finally:
+        stop.append(1)
+        sys.setswitchinterval(before)
+        thread.join()
