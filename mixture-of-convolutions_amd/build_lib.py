@@ -4,12 +4,15 @@ that calls it, _moc_host.so, from csrc/moc_host.cpp with g++ against torch.
     python mixture-of-convolutions_amd/build_lib.py [--jobs N]
 
 Objects go to csrc/_build/, both libraries next to the Python package
-(moc/), where moc/_lib.py loads them.  Every call recompiles.
+(moc/), where moc/_lib.py loads them.  Every call recompiles.  libmoc_hip.so
+needs hipcc only and is linked first; without torch, Python's headers or g++ the
+host module is left out (the Python functions of moc/ then do its calls).
 """
 from __future__ import annotations
 
 import argparse
 import concurrent.futures as cf
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -56,11 +59,26 @@ def _compile(src: Path, extra: tuple[str, ...] = (), build_dir: Path = BUILD) ->
     return obj
 
 
+CXX = os.environ.get("CXX", "g++")
+
+
+def host_needs() -> str | None:
+    """What the host module's build lacks here, or None."""
+    if shutil.which(CXX) is None:
+        return f"a C++ compiler ({CXX})"
+    torch = importlib.util.find_spec("torch")
+    if torch is None or not (Path(torch.origin).parent / "lib" / "libc10_hip.so").exists():
+        return "torch for ROCm"
+    if not (Path(sysconfig.get_path("include")) / "Python.h").exists():
+        return "Python's headers"
+    return None
+
+
 def _compile_host(build_dir: Path) -> Path:
     import torch
     inc = Path(torch.__file__).parent / "include"
     obj = build_dir / "moc_host.o"
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1",
+    cmd = [CXX, "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1",
            "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_moc_host",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f"-I{inc}", f"-I{inc / 'torch/csrc/api/include'}", f"-I{Path(HIPCC).parents[1] / 'include'}",
@@ -75,7 +93,7 @@ def _link_host(obj: Path) -> None:
     import torch
     lib = Path(torch.__file__).parent / "lib"
     tmp = HOST.with_suffix(".so.tmp")
-    cmd = [os.environ.get("CXX", "g++"), "-shared", "-o", str(tmp), str(obj), f"-L{lib}", "-ltorch_python",
+    cmd = [CXX, "-shared", "-o", str(tmp), str(obj), f"-L{lib}", "-ltorch_python",
            "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", f"-L{LIB.parent}",
            f"-l:{LIB.name}", "-Wl,-rpath,$ORIGIN"]
     res = subprocess.run(cmd, capture_output=True, text=True)
@@ -94,19 +112,23 @@ def build(jobs: int | None = None, verbose: bool = True, defines: tuple[str, ...
     sources = sorted(CSRC.glob("*.hip"))
     jobs = jobs or min(len(sources), max(1, (os.cpu_count() or 4)))
     extra = tuple(f"-D{d}" for d in defines)
-    with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
-        host = ex.submit(_compile_host, build_dir) if Path(out) == LIB else None
-        objs = list(ex.map(lambda src: _compile(src, extra, build_dir), sources))
-        host_obj = host.result() if host is not None else None
     LIB_OUT = Path(out)
+    lacks = host_needs() if LIB_OUT == LIB else "not asked for"
+    with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_compile_host, build_dir) if lacks is None else None
+        objs = list(ex.map(lambda src: _compile(src, extra, build_dir), sources))
     tmp = LIB_OUT.with_suffix(".so.tmp")
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + res.stdout + res.stderr)
     os.replace(tmp, LIB_OUT)
-    if host_obj is not None:
-        _link_host(host_obj)
+    if LIB_OUT == LIB:
+        HOST.unlink(missing_ok=True)  # (one of another build of the library)
+        if host is not None:
+            _link_host(host.result())
+        else:
+            print(f"host module not built: needs {lacks}", file=sys.stderr)
     if verbose:
         print(f"built {LIB_OUT} from {len(sources)} sources")
     return LIB_OUT
