@@ -9,6 +9,7 @@ import contextlib
 import ctypes
 import importlib.util
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -213,22 +214,34 @@ HOST_PATH = LIB_PATH.parent / "_moc_host.so"
 _host = None
 
 
+class _NoHost:
+    """In the host module's place where there is none: no call is its own."""
+
+    @staticmethod
+    def _none(*_):
+        return None
+
+    layer = func = stateful = _none
+
+
 def host():
-    """The host module (csrc/moc_host.cpp) on the loaded library; raises
-    RuntimeError if it is not built."""
+    """The host module (csrc/moc_host.cpp) on the loaded library.  It only makes
+    the Python functions' calls cheaper: where it is not built, or built for
+    another torch, they run themselves, and a warning says so once."""
     global _host
     if _host is None:
         lib()
         with _lock:
             if _host is None:
-                if not HOST_PATH.exists():
-                    raise RuntimeError(
-                        f"{HOST_PATH} is not built; run "
-                        "`python mixture-of-convolutions_amd/build_lib.py` "
-                        "(or __graft_entry__.build()) first")
-                spec = importlib.util.spec_from_file_location("_moc_host", HOST_PATH)
-                module = importlib.util.module_from_spec(spec)
-                spec.loader.exec_module(module)
+                try:
+                    spec = importlib.util.spec_from_file_location("_moc_host", HOST_PATH)
+                    module = importlib.util.module_from_spec(spec)
+                    spec.loader.exec_module(module)
+                except (ImportError, OSError) as e:
+                    warnings.warn(f"{HOST_PATH.name} cannot be loaded ({e}); calls are made from Python. "
+                                  "Build it with `python mixture-of-convolutions_amd/build_lib.py`",
+                                  RuntimeWarning, stacklevel=3)
+                    module = _NoHost
                 _host = module
     return _host
 

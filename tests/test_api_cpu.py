@@ -5,12 +5,13 @@ final-state bookkeeping."""
 from __future__ import annotations
 
 import math
+import warnings
 
 import pytest
 import torch
 
 import moc
-from moc import api, ops
+from moc import _lib, api, ops
 
 
 def test_exports():
@@ -208,3 +209,22 @@ def test_group_construction_and_arguments():
     assert not ops.router_grouped_supported(z, [q.router, k.router])
     with pytest.raises(ValueError, match="must all be CUDA tensors"):
         grp(xs, z)
+
+
+@pytest.mark.parametrize("content", [None, b"no library"])
+def test_missing_host_module(tmp_path, monkeypatch, content):
+    """Without a host module that loads, its calls are nobody's, said once: the
+    Python functions run."""
+    path = tmp_path / "_moc_host.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setattr(_lib, "HOST_PATH", path)
+    with pytest.warns(RuntimeWarning, match="_moc_host.so"):
+        H = _lib.host()
+    x = torch.zeros(1, 2, 4)
+    assert H.layer(x, x, x, x, 0, 1, None) is None and H.func(x, x, x, 0, None) is None
+    assert H.stateful(x, x, x, x, None, 0, 1, True) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.host() is H
