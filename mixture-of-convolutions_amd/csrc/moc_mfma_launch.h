@@ -245,11 +245,16 @@ inline Grid2 bwd_taps_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int n_cu
 // tiers of the grids above (two workgroups per CU for its four-wave form, one for
 // the two-wave form), but counted in steps of 32 rows of which a range gives up
 // S - 1 in all (n steps own 32 n - (S - 1) rows; range by starts at row
-// 32 steps_before - by (S - 1)).  Every range has at least one step: there are
-// at most ceil(N / (32 - (S - 1))) ranges.
+// 32 steps_before - by (S - 1)).  Ranges are counted by the rows a step owns alone,
+// 32 - (S - 1): counted by 32 (as the taps pass counts, whose super-blocks own all
+// their rows) the S - 1 rows of each range added up to a second step in some of
+// them, and a grid below one round of workgroups took twice a step (bf16, 32 routes,
+// 2 taps, 2000 tokens, D 128: 63 ranges of 1 or 2 steps 15.4 us, 65 of one 12.5).
+// Every range has at least one step: there are at most ceil(N / (32 - (S - 1))).
 inline Grid2 bwd_lean_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int KC, bool bf, int n_cu) {
   const bool four = lean_waves(static_cast<int>(S), KC, bf) == 4;
-  Grid2 g = four ? bwd_grid_tiered(N, gx, D, S, n_cu) : bwd_taps_grid(N, gx, D, S, n_cu);
+  Grid2 g = four ? bwd_grid_tiered(N, gx, D, S, n_cu)
+                 : bwd_grid_gx(N, gx, D, S, n_cu > 0 ? n_cu : kBwdTargetWG / 2);
   const int64_t gy = g.gy, gy1 = g.gy1;
   const int64_t steps = cdiv(N + gy * (S - 1), 16 * kBwdNB);
   const int64_t n_old = (steps * kBwdOldShare + 50) / 100;

@@ -48,7 +48,7 @@ def bwd_grid_gx(N, gx, D, S, target, taps=False):
 
 def tiered(N, gx, D, S, n_cu, share=62):
     g = bwd_grid_gx(N, gx, D, S, 512)
-    if n_cu % g["gx"]:
+    if n_cu <= 0 or n_cu % g["gx"]:
         return g
     gy1 = n_cu // g["gx"]
     if g["gy"] != 2 * gy1:
@@ -57,9 +57,24 @@ def tiered(N, gx, D, S, n_cu, share=62):
     n_super = cdiv(N, eown)
     n_old = (n_super * share + 50) // 100
     n1, n2 = cdiv(n_old, gy1), cdiv(n_super - n_old, g["gy"] - gy1)
-    if n2 < 1 or n2 > n1:
+    if n1 > ((1 << 30) // (D * 4) - 32) // eown or n2 < 1 or n2 > n1:
         return g
     return dict(g, n_sb=n1, gy1=gy1, n_old=n_old, n_total=n_super)
+
+
+def lean_grid(N, gx, D, S, KC, bf, n_cu, share=62):
+    """bwd_lean_grid: the ranges of the grids above, in 32-row steps of which a
+    range gives up S - 1 rows in all."""
+    if bf and S <= 4 and KC == 1:
+        g = tiered(N, gx, D, S, n_cu, share)
+    else:
+        g = bwd_grid_gx(N, gx, D, S, n_cu or 256)
+    gy, gy1 = g["gy"], g["gy1"]
+    steps = cdiv(N + gy * (S - 1), 32)
+    n_old = (steps * share + 50) // 100
+    if not (gy1 < gy and n_old >= gy1 and steps - n_old >= gy - gy1):
+        gy1, n_old = gy, steps
+    return dict(gx=gx, gy=gy, gy1=gy1, n_old=n_old, n_total=steps)
 
 
 def sb_range(by, g):
