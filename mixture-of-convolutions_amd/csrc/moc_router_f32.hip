@@ -4,13 +4,12 @@
 //
 // All three products have at most 32 routes on one side, so what bounds them is
 // one pass over z (and dz) through HBM; a library GEMM tiles for a wide second
-// side instead (its drouter product ran 38.6 us for 33.5 MB of z).  The products
-// run on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32: 2 N Z K flops each,
-// a fifth of the streaming time at 16 routes), operands are read with 16-byte
-// accesses in the order the instruction wants them (a contraction may be taken
-// in any order if both operands agree: step v of four takes entries 4 q + v), sums
-// are fp32 and in a fixed order.  N 8192, Z 1024, 16 routes: forward with the
-// softmax 14.4 -> 8.6 us, dz and drouter 50.5 -> 16.9 us (library GEMMs before).
+// side instead.  The products run on the fp32 matrix instruction
+// (v_mfma_f32_16x16x4_f32: 2 N Z K flops each, a fifth of the streaming time at 16
+// routes, half of it at 32), a contraction in any order both operands agree on
+// (step v of four takes entries 4 q + v); sums are fp32 and in a fixed order.
+// N 8192, Z 1024, 16 routes, us (a copy of z 13.6): forward with the softmax 10.7,
+// the library's 16.0; dz and drouter 22.9, the library's 51.5.
 // K % 4 == 0, K <= 32, Z % 64 == 0.
 
 #include "moc_kernels.h"
@@ -36,75 +35,112 @@ __device__ __forceinline__ f32x4 mma4(f32x4 a, f32x4 b, f32x4 c) {
 }
 
 // ---------------------------------------------------------------------------
-// out[t, k] = activation_k(sum_z z[t, z] router[k, z]).  Workgroup: 16 tokens, 4
-// waves; wave w sums the 64-wide z chunks w, w + 4, ... with lane (i, q) holding
-// columns 16 u + 4 q + {0..3} (u < 4) of token t0 + i and of route 16 kc + i.  The
-// waves' tiles are summed in LDS in wave order; 16 or 32 consecutive lanes then
-// hold a token's routes and form the activation as the operand preparation
-// forms it (moc_mfma_common.hip).
-template <int KC>
-__global__ void __launch_bounds__(256)
+// out[t, k] = activation_k(sum_z z[t, z] router[k, z]).  Workgroup: 16 tokens, W
+// waves; wave w sums the 64-wide z chunks w, w + W, ...  A product's lane (i, q)
+// wants 16 bytes of row i, but four neighbouring lanes in four rows cost the
+// access path four times what 64 bytes of one row do (16 bytes a clock and CU,
+// whatever the stride or the number of waves: what bounded this kernel).  So a
+// half chunk's tiles (the tokens', and one per 16 routes) are loaded eight lanes
+// to a row of 128 bytes, written to a wave-private LDS tile and read back as
+// operands, while the next chunk's same half is loaded.  The waves' sums are
+// added in pairs, through LDS; 16 or 32 consecutive lanes then hold a token's routes
+// and form the activation as the operand preparation forms it (moc_mfma_common.hip).
+//
+// Us, operands loaded as they lie -> here: 16 routes, Z 1024, 48 tokens 5.6 -> 3.8,
+// 8192 tokens 11.9 -> 11.5; Z 4096, 300 tokens 16.4 -> 8.4, 16384 tokens 68.6 -> 59.1;
+// 32 routes, Z 4096, 48 tokens 23.9 -> 12.8, 16384 tokens 97.9 -> 66.5 (z alone 52 at the
+// copy rate; a library GEMM 55); Z 512, 16384 tokens 16.0 -> 12.1.  Whole chunks in LDS:
+// the same at 16 routes, 14.7 there (fewer workgroups of a CU).  Blocks of 32 tokens
+// (half the reads of the router): half again slower up to 4096 tokens, within 10% past.
+template <int KC, int W>
+__global__ void __launch_bounds__(64 * W)
 router_f32_fwd_kernel(const float* __restrict__ z, const float* __restrict__ r,
                       float* __restrict__ out, int64_t N, int Z, int K, int routing) {
-  constexpr int KP = 16 * KC;
-  __shared__ float red[4][16][KP + 1];
+  constexpr int KP = 16 * KC, T = 1 + KC;  // tiles of a chunk: tokens, routes
+  __shared__ __align__(16) f32x4 st[W][T][128];
+  float(*red)[16][KP + 1] = reinterpret_cast<float(*)[16][KP + 1]>(st);
+  static_assert(sizeof(float) * W * 16 * (KP + 1) <= sizeof(st), "the sums fit the tiles");
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int i = lane & 15, q = lane >> 4;
   const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 16;
   const int64_t rows = N - t0 < 16 ? N - t0 : 16;
+  const int k0 = KP * static_cast<int>(blockIdx.y);  // (first route of this workgroup)
   // rows past N and routes past K lie outside the buffers and load zeros
   const Buf zb(z + t0 * Z, rows * Z * 4);
-  const Buf rb(r, static_cast<int64_t>(K) * Z * 4);
+  const Buf rb(r + static_cast<int64_t>(k0) * Z, static_cast<int64_t>(K - k0) * Z * 4);
   const int nchunk = Z / 64;
-  // one sum per 16 columns of a chunk: chains a quarter as long, for the products
-  // in flight and for the rounding of the sums (Z 1024: 1.55e-7 off the 64-bit
-  // logits, a library GEMM 2.9e-7; a decode step's y 2.4e-7 -> 1.6e-7)
-  f32x4 acc[4][KC];
+  // several sums, each of its 16-column parts of the chunks: short chains, for the
+  // products in flight and for the rounding of the sums (Z 1024: 1.55e-7 off the
+  // 64-bit logits, a library GEMM 2.9e-7; a decode step's y 2.4e-7 -> 1.6e-7)
+  constexpr int US = 16 / W;
+  f32x4 acc[US][KC];
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
+  for (int u = 0; u < US; ++u)
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) acc[u][kc] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // two chunks in flight (a chunk past the row loads zeros)
-  struct Ops {
-    f32x4 z[4], r[KC][4];
-  };
-  auto load = [&](int c, Ops& o) {
+  // load l of a half tile: row 8 l + lane / 8, of its 32 columns the 16 bytes
+  // (lane % 8) ^ (row / 2), to slot 64 l + lane: the 16 rows that a group of lanes
+  // reads then lie in 16 different slots modulo 16
+  uint32_t off[2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const uint32_t col = static_cast<uint32_t>((64 * c + 16 * u + 4 * q) * 4);
-      o.z[u] = load4(zb, c < nchunk ? static_cast<uint32_t>(i * Z * 4) + col : kOffNone);
-#pragma unroll
-      for (int kc = 0; kc < KC; ++kc)
-        o.r[kc][u] = load4(rb, c < nchunk ? static_cast<uint32_t>((16 * kc + i) * Z * 4) + col : kOffNone);
-    }
-  };
-  auto mult = [&](const Ops& o) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int kc = 0; kc < KC; ++kc) acc[u][kc] = mma4(o.z[u], o.r[kc][u], acc[u][kc]);
-  };
-  Ops a, b;
-  load(w, a);
-  for (int c = w; c < nchunk; c += 8) {
-    load(c + 4, b);
-    mult(a);
-    load(c + 8, a);
-    mult(b);
+  for (int l = 0; l < 2; ++l) {
+    const int row = 8 * l + (lane >> 3);
+    off[l] = (static_cast<uint32_t>(row) * Z + 4 * ((lane & 7) ^ (row >> 1))) * 4;
   }
+  f32x4 raw[2][T][2];
+  auto load = [&](int c, int h) {  // (a chunk past the row loads zeros)
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int l = 0; l < 2; ++l) {
+        const uint32_t tile = static_cast<uint32_t>(t > 0 ? 16 * (t - 1) : 0) * Z * 4 + 256 * c + 128 * h;
+        raw[h][t][l] = load4(t > 0 ? rb : zb, c < nchunk ? off[l] + tile : kOffNone);
+      }
+  };
+  load(w, 0);
+  load(w, 1);
+  for (int c = w; c < nchunk; c += W) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int l = 0; l < 2; ++l) st[w][t][64 * l + lane] = raw[h][t][l];
+      load(c + W, h);
+      __builtin_amdgcn_sched_barrier(0);
+      mfma::wave_lds_sync();
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        // row i, columns 32 h + 16 u + 4 q + {0..3}
+        const int slot = 64 * (i >> 3) + 8 * (i & 7) + ((4 * u + q) ^ (i >> 1)), a = (2 * h + u) % US;
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) acc[a][kc] = mma4(st[w][0][slot], st[w][1 + kc][slot], acc[a][kc]);
+      }
+      mfma::wave_lds_sync();
+    }
+  }
+  __syncthreads();
   // D lane (j, q): route 16 kc + j, tokens 4 q + v
 #pragma unroll
   for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-      red[w][4 * q + v][16 * kc + i] = (acc[0][kc][v] + acc[1][kc][v]) + (acc[2][kc][v] + acc[3][kc][v]);
+    for (int v = 0; v < 4; ++v) {
+      float s = acc[0][kc][v] + acc[1][kc][v];
+      if constexpr (US == 4) s += acc[2][kc][v] + acc[3][kc][v];
+      red[w][4 * q + v][16 * kc + i] = s;
+    }
   __syncthreads();
-#pragma unroll
-  for (int pass = 0; pass < KC; ++pass) {
-    const int idx = threadIdx.x + 256 * pass;
+  for (int idx = threadIdx.x; idx < 16 * KP; idx += 64 * W) {  // (whole waves: 16 KP is 4 or 8 of them)
     const int tok = idx / KP, k = idx % KP;
-    float v = ((red[0][tok][k] + red[1][tok][k]) + red[2][tok][k]) + red[3][tok][k];
+    float part[W];
+#pragma unroll
+    for (int ww = 0; ww < W; ++ww) part[ww] = red[ww][tok][k];
+#pragma unroll
+    for (int d = 1; d < W; d *= 2)
+#pragma unroll
+      for (int ww = 0; ww < W; ww += 2 * d) part[ww] += part[ww + d];
+    float v = part[0];
     if (routing == ROUTE_SOFTMAX) {
       const float l = k < K ? v : -INFINITY;
       float m = l;
@@ -118,7 +154,7 @@ router_f32_fwd_kernel(const float* __restrict__ z, const float* __restrict__ r,
     } else if (routing == ROUTE_EXP) {
       v = __expf(v);
     }
-    if (k < K && tok < rows) out[(t0 + tok) * K + k] = v;
+    if (k0 + k < K && tok < rows) out[(t0 + tok) * K + k0 + k] = v;
   }
 }
 
@@ -279,8 +315,20 @@ bool router_f32_supported(int64_t N, int64_t Z, int64_t K) {
 
 void router_f32_forward(const void* z, const void* r, void* out, int64_t N, int64_t Z, int64_t K,
                         int routing, hipStream_t st) {
-  auto kern = K <= 16 ? router::router_f32_fwd_kernel<1> : router::router_f32_fwd_kernel<2>;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(router::cdiv(N, 16))), dim3(256), 0, st,
+  // eight waves a workgroup while every CU has at most one and each wave a chunk, else
+  // four (16 routes, Z 4096, 2000 tokens: 12.3 us with eight, 15.3 with four; 32 routes,
+  // Z 512, 16384 tokens: 13.9 and 12.1; below Z 512 four waves' shorter sums are 20%
+  // closer to 64 bits for 0.4 us)
+  const int64_t blocks = router::cdiv(N, 16);
+  const bool eight = blocks <= 256 && Z >= 512;
+  // more than 16 routes in two workgroups of 16 where half the CUs would be idle and
+  // no softmax joins them: a CU's matrix rate bounds a token block (decode step of 16
+  // tokens, Z 4096, 32 routes: its router 12.8 -> 8.0 us)
+  const bool halves = K > 16 && routing != ROUTE_SOFTMAX && 2 * blocks <= 256;
+  const bool one = K <= 16 || halves;
+  auto kern = one ? (eight ? router::router_f32_fwd_kernel<1, 8> : router::router_f32_fwd_kernel<1, 4>)
+                  : (eight ? router::router_f32_fwd_kernel<2, 8> : router::router_f32_fwd_kernel<2, 4>);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(blocks), halves ? 2 : 1), dim3(eight ? 512 : 256), 0, st,
                      static_cast<const float*>(z), static_cast<const float*>(r),
                      static_cast<float*>(out), N, static_cast<int>(Z), static_cast<int>(K), routing);
 }
