@@ -301,6 +301,19 @@ OptTensor func(const Tensor& x, const Tensor& alpha, const Tensor& basis, int ac
   return run_forward(c, x.contiguous(), alpha.contiguous(), basis.contiguous(), 0);
 }
 
+// Whether a prompt's state is cheaper written by the forward launch than as a copy of
+// its last rows after the plain forward.  It saves a launch and a slow transposed copy
+// (bf16, 8 x 1024 tokens, D 2048, 16 routes, 4 taps: 27 -> 22 us), but the kernel with
+// a cache to read walks a sequence's first S - 1 rows one tap at a time (8 taps, 8 x 3
+// tokens: 6.3 us plain, 18.9), and in fp32 its larger tile costs more than the copy
+// from about 2^22 elements on with more than 3 taps or 16 routes (8 x 2048 tokens, D
+// 4096, 4 taps, 16 routes 126 -> 141; 6 taps, 32 routes 256 -> 309; 3 x 300 tokens, D
+// 1544, 4 taps 12 -> 10).
+bool state_in_forward(const Call& c) {
+  if (c.T < c.S - 1) return false;
+  return c.dt == 1 || c.N * c.D <= (int64_t(1) << 22) || (c.S <= 3 && c.K <= 16);
+}
+
 // (y, state or None) of MoC.forward with a cache or a final state, fixed length:
 // one token per sequence and a cache: the decode step, in place on the cache
 // (not differentiable); else without gradients only.  Nothing: not a call of
@@ -339,6 +352,7 @@ std::optional<std::tuple<Tensor, OptTensor>> stateful(const Tensor& x, const Ten
   }
   if (wants_grad({&x, &z, &router, &basis, cache.has_value() ? &*cache : nullptr})) return std::nullopt;
   if (!moc_prefill_supported(B, c.T, c.D, c.K, c.S, c.dt, cache.has_value())) return std::nullopt;
+  if (!cache.has_value() && !state_in_forward(c)) return std::nullopt;
   at::NoGradGuard ng;
   const Tensor xc = x.contiguous(), bc = basis.contiguous();
   const Tensor w = run_router(c, z.contiguous(), router.contiguous(), route);

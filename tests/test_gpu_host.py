@@ -198,6 +198,24 @@ def test_stateful_bit_for_bit(dtype):
         assert (y - ref).float().abs().max() <= 2.0 ** -7 * ref.float().abs().max()
 
 
+@pytest.mark.parametrize("dtype,B,T,D,K,S,one", [
+    (BF, 2, 2, 130, 16, 4, False), (BF, 2, 3, 130, 16, 4, True), (BF, 3, 6, 130, 32, 8, False),
+    (F32, 2, 7, 130, 16, 8, True), (F32, 1, 1024, 4096, 16, 4, True), (F32, 1, 1025, 4096, 16, 4, False),
+    (F32, 1, 1025, 4096, 16, 3, True), (F32, 2, 600, 4098, 20, 3, False), (BF, 1, 1025, 4096, 32, 8, True)])
+def test_prompt_state(dtype, B, T, D, K, S, one):
+    """A prompt's state from the forward launch, or the plain forward's rows where
+    those are cheaper: the same y and state."""
+    m, g = _layer(dtype, K, S, D), gen(T)
+    x, z = randn(g, B, T, D).to(DEV, dtype), randn(g, B, T, 128).to(DEV, dtype)
+    with torch.no_grad():
+        out = _lib.host().stateful(x, z, m.router, m.conv_bases, None, 1, 1, True)
+        assert (out is not None) == one
+        y, state = m(x, z, output_final_state=True)
+        w = api.ops.router_forward(z, m.router, routing=1)
+        ref = api.ops.launch_forward(x, w, m.conv_bases, activation_flag=1, routing=3)
+    assert torch.equal(y, ref) and torch.equal(state, api._final_state(x, None, S))
+
+
 def _step(m, x, z, dy):
     y, _ = m(x, z)
     return [y.detach(), *torch.autograd.grad(y, [x, z, m.router, m.conv_bases], dy)]
