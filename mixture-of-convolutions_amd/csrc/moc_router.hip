@@ -12,7 +12,7 @@
 // activation K <= 32), Z % 64 == 0.
 
 #include "moc_kernels.h"
-#include "moc_mfma.h"
+#include "moc_mfma_launch.h"
 
 namespace moc {
 namespace router {
@@ -54,8 +54,8 @@ __device__ __forceinline__ s16x4 tr_read(const void* p) {
 
 // ---------------------------------------------------------------------------
 // logits[t, k] = sum_z z[t, z] router[k, z].  Workgroup: HB blocks of 16 tokens
-// (two; four with more than 32 routes and rows enough: below), 4 waves.  Wave w sums the 64-wide z chunks c = w, w + 4, ...: lane
-// (i, qq) loads columns 64 c + 8 qq + [0, 8) and 64 c + 32 + 8 qq + [0, 8) of
+// (two; four with more than 32 routes and rows enough: FwdLaunch), 4 waves.  Wave w
+// sums the 64-wide z chunks c = w, w + 4, ...: lane (i, qq) loads columns 64 c + 8 qq + [0, 8) and 64 c + 32 + 8 qq + [0, 8) of
 // tokens t0 + 16 h + i (A operands) and of route 16 kc + i (B operands),
 // so that each load instruction reads 64 contiguous bytes per row and the
 // router operands serve every token block.  The 4 partial tiles are summed in
@@ -63,8 +63,7 @@ __device__ __forceinline__ s16x4 tr_read(const void* p) {
 // Two token blocks re-read the whole router from L2 for every 32 rows of z (96
 // routes, Z 4096: 402 MB of it beside 134 MB of z at N 16384, 67 us); four halve
 // that (45.5 us), a wave per SIMD with up to 256 VGPRs holding the next round's
-// loads.  Up to 32 routes the router is the smaller part, and below 64 x 256
-// rows (one workgroup for each of 256 CUs) the smaller workgroups fill the chip.
+// loads.  Up to 32 routes the router is the smaller part.
 // Chunks whose loads are issued together: four up to 32 routes, fewer above
 // (the router operands of a chunk take 8 KC registers per lane).
 template <int KC>
@@ -786,8 +785,14 @@ struct FwdLaunch {
                   int routing, const RouteGroups& grp, hipStream_t st) {
     const dim3 grid(static_cast<unsigned>(cdiv(N, 32)));
     if constexpr (KC > 2) {
-      // the four-block form where it gives every one of 256 CUs a workgroup
-      if (N >= 64 * 256) {
+      // the four-block form where it gives every CU a workgroup and the loop is long
+      // enough to pay for its larger sums (us, two blocks -> four, N 20000: 96 routes, Z
+      // 64 7.5 -> 10.8, Z 512 16.6 -> 19.3, Z 1024 27.9 -> 28.8, Z 2048 50.4 -> 47.9; N
+      // 16384: Z 512 12.4 -> 11.2, Z 1024 20.0 -> 16.6, Z 4096 66.1 -> 47.2; N 32768: Z 512
+      // 22.3 -> 21.2, Z 1024 36.4 -> 31.7; 48 routes, N 20000: Z 512 10.4 -> 10.8, Z 1024 20.1
+      // -> 18.9)
+      const int cus = mfma::device_cu_count();
+      if (Z >= 1024 && N >= int64_t(64) * (cus > 0 ? cus : 256)) {
         const dim3 grid4(static_cast<unsigned>(cdiv(N, 64)));
         if (grp.n > 0)
           hipLaunchKernelGGL((router_fwd_kernel<KC, true, 4>), grid4, dim3(256), 0, st, z, r, out, N, Z,

@@ -73,6 +73,13 @@ def test_router_many_routes_many_tokens(N, Z, Ks):
     assert_close("drouter", dr, dl.float().T @ z.float(), BF)
 
 
+# z_dim and token count at and below the line of the 64-token forward
+@pytest.mark.parametrize("N,Z,Ks", [(16384, 1024, (16, 32)), (16447, 1088, (32, 32, 32)), (16384, 960, (32, 32)),
+                                    (16383, 1024, (32, 20))])
+def test_router_many_routes_forward_forms(N, Z, Ks):
+    test_router_many_routes_many_tokens(N, Z, Ks)
+
+
 def test_router_batched_input_and_autograd():
     B, T, Z, K = 3, 37, 128, 16
     g = gen(5)
