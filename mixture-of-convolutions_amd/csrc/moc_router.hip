@@ -880,8 +880,13 @@ void router_backward(const void* z, const void* r, const void* dl, void* dz, voi
   const int Zi = static_cast<int>(Z), Ki = static_cast<int>(K);
   const router::BwdPlan pl = router::bwd_plan(N, Z);
   float* part = static_cast<float*>(workspace);
-  // both outputs: one pass over z and dz
-  if (dz != nullptr && dr != nullptr) {
+  // both outputs: one pass over z and dz, but for 33 to 48 routes between 2^25 and 5 2^24
+  // elements of z the two launches (same bits; us, one pass against them, 48 routes:
+  // 2000 x 2048 14.3 / 20.6, 2^24 27.6 / 28.4, 8192 x 4096 43.2 / 41.3, 16384 x 2048 44.6 /
+  // 43.3, 16384 x 4096 75.8 / 71.2, 65536 x 1024 78.7 / 74.2, 20000 x 4096 92.9 / 92.4, 32768 x
+  // 4096 151.8 / 162.0; 64 routes: one pass at every size)
+  const bool apart = K > 32 && K <= 48 && N * Z >= (int64_t(1) << 25) && N * Z < (int64_t(5) << 24);
+  if (dz != nullptr && dr != nullptr && !apart) {
     router::with_kc<router::BwdLaunch>(K, dp, zp, rp, static_cast<uint16_t*>(dz), part, N, Zi, Ki, pl, st);
     router::dr_reduce(part, dr, K, Z, pl, st);
     return;

@@ -73,9 +73,11 @@ def test_router_many_routes_many_tokens(N, Z, Ks):
     assert_close("drouter", dr, dl.float().T @ z.float(), BF)
 
 
-# z_dim and token count at and below the line of the 64-token forward
+# z_dim and token count at and below the line of the 64-token forward, and of the backward's
+# two launches
 @pytest.mark.parametrize("N,Z,Ks", [(16384, 1024, (16, 32)), (16447, 1088, (32, 32, 32)), (16384, 960, (32, 32)),
-                                    (16383, 1024, (32, 20))])
+                                    (16383, 1024, (32, 20)),
+                                    (32768, 1024, (16, 16, 16)), (32767, 1024, (32, 16))])
 def test_router_many_routes_forward_forms(N, Z, Ks):
     test_router_many_routes_many_tokens(N, Z, Ks)
 
