@@ -220,28 +220,206 @@ def test_bwd_tile_lds_extents(S, KC, MODE, SPLIT):
     assert len(seen) == NB * KX * 256
 
 
-def test_lean_lds_extents():
-    """bwd_lean_tile: the two row-shifted copies of the routing weights (W
-    operand reads at shift e < 4 stay within an 8-row group, so the swizzle of
-    the row equals that of the lane's base row), transposed alpha reads, m tile
-    and dalpha tiles."""
-    R, TB, KP = 8, 32, 16
-    for S in (2, 3, 4):
-        AROWS = TB + S - 1
-        for j, q in itertools.product(range(16), range(4)):
-            base = R * (j >> 2) + (j & 3)
-            for b, e in itertools.product(range(2), range(S)):  # shifts e < S
-                r = base + e
-                assert r < AROWS - 4 * b  # rows of copy b that were staged
-                assert (r >> 3) == (j >> 2)  # one swizzle over the shifts
-                assert acol(r, 4 * q, KP) == ((q ^ (j >> 2)) << 2)
-            for b in range(2):
-                r = R * q + 4 * b + (j >> 2)
-                assert r < AROWS
-        for tid in range(512):
-            if tid < AROWS * KP // 4:
-                row = tid >> 2
-                assert row < AROWS and (row < 4 or row - 4 < AROWS)
+# ---------------------------------------------------------------------------
+# bwd_lean_tile (csrc/moc_bwd_lean.h): LDS layouts
+
+LEAN = [(bf, KC, S) for bf in (1, 0) for KC in (1, 2) for S in range(2, 9) if bf or KC == 1 or S <= 5]
+F32_ROWS, F32_BASIS = 32 * 16 + 3 * 16, 16 * 16 + 3 * 16
+
+
+def asw(row, KC):
+    return (row >> 3) & 3 if KC == 1 else ((row >> 1) & 1) | (((row >> 3) & 3) << 1)
+
+
+def f32_slot(P, row, chunk, sw):
+    return row * 16 + (row // P) * 16 + 4 * (chunk ^ sw)
+
+
+def f32_aslot(row, chunk):
+    return f32_slot(8, row, chunk, row >> 3)
+
+
+def f32_mslot(row, chunk):
+    return f32_slot(8, row, chunk, (row >> 2) & 3)
+
+
+def f32_bslot(row, chunk):
+    return f32_slot(4, row, chunk, row >> 2)
+
+
+@pytest.mark.parametrize("bf,KC,S", LEAN)
+def test_lean_lds_fits(bf, KC, S):
+    """All of a workgroup's arrays within a CU's 160 KB (half of them for the
+    four-wave form, two workgroups per CU)."""
+    esz, opnd, KP = (2, 8, 16 * KC) if bf else (4, 16, 16 * KC)
+    four = bf and S <= 4 and KC == 1
+    total = 2 * (32 * KP if bf else KC * F32_ROWS) * esz             # a_lds
+    total += (8 if bf else 1) * 2 * 128 * opnd                       # m_tr
+    total += (1 if bf else 8) * F32_ROWS * 4                         # m_f32
+    total += 8 * S * KC * (64 if bf else F32_BASIS // 4) * opnd      # b_lds
+    total += (2 if bf or KC == 1 else 1) * 8 * 2 * KC * 16 * 17 * 4  # da_lds
+    total += ((S - 1) * 512 if four else 1) * 4                      # c0_lds
+    assert total <= 163840 // (2 if four else 1)
+
+
+@pytest.mark.parametrize("KC", [1, 2])
+def test_lean_operands_bf16(KC):
+    """What each lane reads is what the instruction wants there: routing weights
+    and basis tiles as staged and read transposed, m's tile."""
+    lanes = list(itertools.product(range(16), range(4)))
+    # routing weights: slot (row, 4-route chunk) of the staging threads
+    a = {}
+    for t in range(128 * KC):
+        row, c = t // (4 * KC), t % (4 * KC)
+        assert row < 32 and 0 <= c ^ asw(row, KC) < 4 * KC
+        assert a.setdefault((row, c ^ asw(row, KC)), (row, c)) == (row, c)
+    assert len(a) == 32 * 4 * KC
+    for (j, q), b, kc in itertools.product(lanes, range(2), range(KC)):
+        row = 8 * (j >> 2) + 4 * b + (j & 3)
+        assert a[row, (4 * kc + q) ^ asw(row, KC)] == (row, 4 * kc + q)
+    for q, b, kc in itertools.product(range(4), range(2), range(KC)):
+        slots = [a[r, (4 * kc + (j & 3)) ^ asw(r, KC)]
+                 for j in range(16) for r in (8 * q + 4 * b + (j >> 2),)]
+        for i, got in enumerate(tr_read(slots, None)):
+            assert [(row, 4 * c + e) for (row, c), e in got] == \
+                [(8 * q + 4 * b + v, 16 * kc + i) for v in range(4)]
+    # basis: slot of lane (j, q): route j, channels 4 q + {0..3}
+    bt = {}
+    for j, q in lanes:
+        assert bt.setdefault(j * 4 + (q ^ (j >> 2)), (j, q)) == (j, q)
+    assert sorted(bt) == list(range(64))
+    for q in range(4):
+        slots = [bt[(4 * q + (j >> 2)) * 4 + ((j & 3) ^ q)] for j in range(16)]
+        for i, got in enumerate(tr_read(slots, None)):
+            assert [(k, 4 * c + e) for (k, c), e in got] == [(4 * q + v, i) for v in range(4)]
+    # m: writer lane (channel j, stream q), token block b; reader: channels 4 qq + e of token 16 rb + i
+    def wslot(j, q, b):
+        g = 2 * q + b
+        return g * 16 + (j ^ (4 * (g & 3)))
+
+    def rslot(i, qq, rb):
+        e, a4 = i >> 2, i & 3
+        return (4 * rb + a4) * 16 + ((4 * qq + e) ^ (4 * a4))
+
+    m = {wslot(j, q, b): (j, 8 * q + 4 * b) for (j, q), b in itertools.product(lanes, range(2))}
+    assert sorted(m) == list(range(128))
+    for qq, rb in itertools.product(range(4), range(2)):
+        slots = [rslot(i, qq, rb) for i in range(16)]
+        assert len({s % 16 for s in slots}) == 16  # no bank conflict
+        for i, got in enumerate(tr_read([m[s] for s in slots], None)):
+            assert [(ch, tok + e) for (ch, tok), e in got] == [(4 * qq + v, 16 * rb + i) for v in range(4)]
+
+
+def test_lean_operands_f32():
+    """The same of the fp32 tiles: every slot inside its array, one owner, 16-byte
+    reads aligned, each lane's reads what was written there."""
+    tiles = {"a": (f32_aslot, 32, F32_ROWS), "m": (f32_mslot, 32, F32_ROWS), "b": (f32_bslot, 16, F32_BASIS)}
+    held = {}
+    for name, (slot, rows, size) in tiles.items():
+        own = {}
+        for row, c, e in itertools.product(range(rows), range(4), range(4)):
+            at = slot(row, c) + e
+            assert slot(row, c) % 4 == 0 and 0 <= at < size and at not in own
+            own[at] = (row, 4 * c + e)
+        held[name] = own
+    for j, q in itertools.product(range(16), range(4)):
+        for b, v in itertools.product(range(2), range(4)):
+            row = 8 * (j >> 2) + 4 * b + (j & 3)
+            assert held["a"][f32_aslot(row, q) + v] == (row, 4 * q + v)
+            row = 8 * q + 4 * b + v
+            assert held["a"][f32_aslot(row, j >> 2) + (j & 3)] == (row, j)
+            assert held["m"][f32_mslot(16 * b + j, q) + v] == (16 * b + j, 4 * q + v)
+            assert held["b"][f32_bslot(4 * q + v, j >> 2) + (j & 3)] == (4 * q + v, j)
+        for r in range(8):
+            assert held["m"][f32_mslot(8 * q + r, j >> 2) + (j & 3)] == (8 * q + r, j)
+
+
+# ---------------------------------------------------------------------------
+# bwd_lean_tile: rows of the streams, hand-over between them, partials
+
+def lean_rows(N, S, g, by):
+    """What range `by` does with its rows: the rows whose dx it stores with the (t,
+    off) terms of each (dx[t - off] += g[t] W), the rows whose dalpha it stores, the
+    rows whose dbasis products it keeps."""
+    H = S - 1
+    lo, hi = sb_range(by, g)
+    n, first = hi - lo, 32 * lo - by * H
+    end = first + 32 * n
+    own_hi = min(end - H, N)
+    carry = {}   # (stream, row of the stream): terms, the rows -H.. of the next stream's first step included
+    stores, dalpha, dbasis = {}, [], []
+
+    def store(row, terms):
+        if row < own_hi:
+            assert row >= first and row not in stores
+            stores[row] = terms
+
+    owed = {}
+    tail = {}
+    for q in range(4):
+        acc = {w: [] for w in range(-H, 8 * n)}
+        for rho, off in itertools.product(range(8 * n), range(S)):
+            t = first + 8 * n * q + rho
+            if t < N:  # (rows past the last token are masked)
+                acc[rho - off].append((t, off))
+        owed[q] = [acc[w] for w in range(-H, 0)]
+        for i in range(n):
+            for w in range(8):  # rows -(S-1) .. 8-S of the step are complete
+                if w >= H or i > 0:
+                    store(first - H + 8 * n * q + 8 * i + w, acc[8 * i + w - H])
+            for r in range(8):
+                row = first + 8 * n * q + 8 * i + r
+                assert row < end
+                if row < own_hi:
+                    dalpha.append(row)
+                if not (i + 1 == n and q == 3 and r >= 8 - H) and row < N:
+                    dbasis.append(row)
+        tail[q] = [acc[w] for w in range(8 * n - H, 8 * n)]
+    for q, e in itertools.product(range(4), range(H)):
+        store(first - H + 8 * n + e + 8 * n * q, tail[q][e] + owed[(q + 1) % 4][e])
+    return first, own_hi, stores, dalpha, dbasis
+
+
+def lean_cases():
+    for bf, KC, S in LEAN:
+        own = 33 - S
+        for N, D, n_cu in ((1, 2, 256), (own, 130, 256), (own + 1, 130, 256), (8 * own + 3, 130, 256),
+                           (777, 256, 16), (1200, 130, 8)):
+            yield N, D, S, KC, bf, n_cu
+    for S in (2, 3, 4):  # unequal ranges of the two tiers: exactly two workgroups per CU
+        yield 512 * (33 - S) - 5, 130, S, 1, 1, 256
+
+
+def test_lean_rows_and_partials():
+    """Over every range: each row's dx stored once with each of its terms, dalpha
+    stored and dbasis summed once a row; each partial of dbasis written once."""
+    tiers = 0
+    for N, D, S, KC, bf, n_cu in lean_cases():
+        gx = cdiv(D, 128)
+        g = lean_grid(N, gx, D, S, KC, bf, n_cu)
+        tiers += g["gy1"] < g["gy"]
+        dx, da, db, prev = {}, [], [], 0
+        for by in range(g["gy"]):
+            first, own_hi, stores, dalpha, dbasis = lean_rows(N, S, g, by)
+            assert by == 0 or first == prev or first >= N  # a range starts where the last one's own rows end
+            prev = own_hi
+            dx.update(stores)
+            da += dalpha
+            db += dbasis
+        rows = list(range(N))
+        assert sorted(dx) == rows and sorted(da) == rows and sorted(db) == rows, (N, S, KC, bf, n_cu)
+        for u, terms in dx.items():
+            assert sorted(terms) == [(u + off, off) for off in range(S) if u + off < N], (N, S, u)
+        cells = set()
+        for bx, wave, j, q, kc, v in itertools.product(range(gx), range(8), range(16), range(4), range(KC), range(4)):
+            ch = (bx * 8 + wave) * 16 + 4 * q + v
+            if (bx * 8 + wave) * 16 + 4 * q < D and ch < D:
+                assert (16 * kc + j, ch) not in cells
+                cells.add((16 * kc + j, ch))
+        assert len(cells) == 16 * KC * D
+        # the dalpha sums: each of a step's 32 rows and 16 columns by one thread
+        assert len({(t >> 4, t & 15) for t in range(512)}) == 512
+    assert tiers == 3
 
 
 def coverage(N, D, S, KC, mode, SPLIT, n_cu=256):
@@ -300,36 +478,6 @@ def test_partials_written_once(N, D, S, KC, mode, SPLIT, n_cu):
     g = coverage(N, D, S, KC, mode, SPLIT, n_cu)
     if mode == "fused" and not SPLIT and n_cu == 16:
         assert g["gy1"] * 2 == g["gy"] and g["n_old"] < g["n_total"]  # tiers in use
-
-
-def test_lean_partials_written_once():
-    """bwd_lean_tile on the fused pass's (two-tier) grid: 8 waves of 16 channels
-    per 128-channel group, dalpha rows of the own tokens, dbasis (k, s, 4
-    channels per lane)."""
-    for N, D, S, n_cu in ((464, 256, 4, 16), (999, 196, 3, 256), (77, 64, 2, 256)):
-        KP, eown = 16, 32 - (S - 1)
-        g = tiered(N, cdiv(D, 128), D, S, n_cu)
-        da, db = {}, {}
-        for bx, by, _ in blocks(g, 1):
-            lo, hi = sb_range(by, g)
-            for sb in range(lo, hi):
-                t0 = sb * eown
-                if t0 >= N:
-                    break
-                own = min(t0 + eown, N) - t0
-                for tl in range(512):
-                    r2, row, c = tl >> 8, (tl >> 4) & 15, tl & 15
-                    if 16 * r2 + row < own:
-                        key = (bx, t0 + 16 * r2 + row, c)
-                        da[key] = da.get(key, 0) + 1
-            for wave, j, q, s, v in itertools.product(range(8), range(16), range(4), range(S),
-                                                      range(4)):
-                d0 = (bx * 8 + wave) * 16
-                if d0 < D and d0 + 4 * q < D:
-                    key = (by, j, s, d0 + 4 * q + v)
-                    db[key] = db.get(key, 0) + 1
-        assert all(n == 1 for n in da.values()) and len(da) == g["gx"] * N * KP
-        assert all(n == 1 for n in db.values()) and len(db) == g["gy"] * KP * S * D
 
 
 # ---------------------------------------------------------------------------
