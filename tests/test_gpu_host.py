@@ -9,6 +9,7 @@ import time
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import moc
 from moc import MoC, api
@@ -142,9 +143,20 @@ def test_watched_calls_stay_with_python():
         assert H.layer(torch.autograd.forward_ad.make_dual(x, x), z, *args) is None
     inside = []
     torch.func.vmap(lambda t: (inside.append(H.layer(t[None], z[:1], *args)), t)[1])(x)
-    torch.func.grad(lambda t: (inside.append(H.layer(t, z, *args)), t.sum().float())[1])(x.float())
+    torch.func.grad(lambda t: (inside.append(H.layer(t, z, *args)), t.sum())[1])(x)
     torch.jit.trace(lambda t: (inside.append(H.layer(t, z, *args)), t)[1], (x,), check_trace=False)
-    assert inside and all(v is None for v in inside)
+    class Seen(TorchDispatchMode):
+        ops = 0
+
+        def __torch_dispatch__(self, func, types, call, kwargs=None):
+            self.ops += 1
+            return func(*call, **(kwargs or {}))
+
+    with Seen() as seen:
+        inside.append(H.layer(x, z, *args))
+        y, _ = m(x, z)
+    assert seen.ops > 0 and torch.equal(y, m(x, z)[0])
+    assert len(inside) == 4 and all(v is None for v in inside)
     assert H.layer(x.cpu(), z, *args) is None and H.layer(x.half(), z, *args) is None
     assert H.layer(x[:, :0], z[:, :0], *args) is None and H.layer(x, z[:, :5], *args) is None
 
@@ -195,7 +207,10 @@ def test_stateful_bit_for_bit(dtype):
         ref = api._step(x[:, :1], logits, m.conv_bases, one, "silu", "softmax")
         y, out = m.step(x[:, :1], z[:, :1], cache=two, output_final_state=True)
         assert out is two and torch.equal(one, two)
-        assert (y - ref).float().abs().max() <= 2.0 ** -7 * ref.float().abs().max()
+        if dtype == F32:  # the same two launches
+            assert torch.equal(y, ref)
+        else:  # the one-launch step rounds its weights as another kernel does
+            assert (y - ref).float().abs().max() <= 2.0 ** -7 * ref.float().abs().max()
 
 
 @pytest.mark.parametrize("dtype,B,T,D,K,S,one", [

@@ -51,13 +51,30 @@ def test_stream_edges_fixed(S, K, act, B, T, D):
                                      (8, 32, None)])
 @pytest.mark.parametrize("longest", [3, 45, 700])
 def test_stream_ranges_packed(S, K, act, longest):
-    # 256 ranges (128 of the two-wave form) of the two 128-channel groups; two to
-    # five steps each
+    # on 256 CUs 172 to 249 ranges of the two 128-channel groups, one to three steps each,
+    # in the four-wave form, 103 to 120 of four or five in the two-wave form
     g = gen(S * 10 + longest)
     N, D = 256 * 29 * 2 + 77, 130
     lengths, left = [], N
     while left:
         n = min(left, int(torch.randint(1, longest + 1, (1,), generator=g)))
+        lengths.append(n)
+        left -= n
+    _check(randn(g, N, D, scale=0.5), torch.softmax(randn(g, N, K), -1),
+           randn(g, K, S, D, scale=0.3), randn(g, N, D), act, lengths)
+
+
+@pytest.mark.parametrize("S,K,act", [(2, 12, "silu"), (2, 16, None), (3, 12, "silu"), (4, 12, None),
+                                     (4, 16, "silu")])
+@pytest.mark.parametrize("longest", [0, 3, 700])
+def test_stream_two_tiers(S, K, act, longest):
+    # on 256 CUs two workgroups per CU of the two channel groups exactly: 256 ranges, the
+    # first half of them longer (0: one sequence)
+    g = gen(S * 20 + longest)
+    N, D = 512 * (33 - S) - 5, 130
+    lengths, left = [], N
+    while left:
+        n = min(left, int(torch.randint(1, longest + 1, (1,), generator=g))) if longest else N
         lengths.append(n)
         left -= n
     _check(randn(g, N, D, scale=0.5), torch.softmax(randn(g, N, K), -1),
@@ -90,7 +107,7 @@ def test_stream_edges_fixed_f32(S, K, act, B, T, D):
                                      (4, 32, "silu"), (5, 20, None)])
 @pytest.mark.parametrize("longest", [3, 700])
 def test_stream_ranges_packed_f32(S, K, act, longest):
-    # 128 ranges of the two channel groups, two to four steps each
+    # on 256 CUs 97 to 121 ranges of the two channel groups, two to four steps each
     g = gen(S * 10 + longest)
     N, D = 128 * 29 * 3 + 77, 130
     lengths, left = [], N
