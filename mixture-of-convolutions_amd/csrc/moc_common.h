@@ -118,8 +118,9 @@ struct SeqLayout {
   }
 
   // Smallest segment start >= lo (segment starts: 0, the cu entries, in order),
-  // or n_tokens if there is none below n_tokens.  Called with wave-uniform
-  // arguments, so its loads are scalar.
+  // or n_tokens if there is none below n_tokens.  (With wave-uniform arguments its
+  // loads are scalar; the stream backward calls it per lane, each lane group's rows
+  // being a stream of their own, once per segment that a stream passes.)
   __device__ __forceinline__ int64_t next_start(int64_t lo) const {
     if (lo <= 0) return 0;
     if (lo >= n_tokens) return n_tokens;

@@ -755,15 +755,20 @@ bool layers_grouped(const Problem* ps, int n, bool backward) {
 
 namespace {
 // Stage-1 class of a layer in a grouped backward: its route chunks, and its
-// activation where either activation's layers run a two-pass form, or only one
-// of them the lean pass (different forms cannot share a launch).
+// activation where either activation's layers run a two-pass form (different
+// forms cannot share a launch; the lean pass takes both).
+constexpr bool lean_of_either_activation() {
+  for (int S = 2; S <= 8; ++S)
+    for (int KC = 1; KC <= 4; KC *= 2)
+      if (bwd_lean(S, KC, false, true) != bwd_lean(S, KC, true, true)) return false;
+  return true;
+}
+static_assert(lean_of_either_activation(), "a class of lean layers holds both activations");
 int bwd_class(const Problem& p) {
   const int S = static_cast<int>(p.S), KC = route_chunks(p.K);
-  const bool lean0 = bwd_lean(S, KC, false, true);
-  const bool lean1 = bwd_lean(S, KC, true, true);
-  const bool two = lean0 != lean1 ||
-                   (!lean0 && (bwd_two_pass(S, KC, false, true) || bwd_two_pass_r(S, KC, false, true) ||
-                               bwd_two_pass_g(S, KC, true, true)));
+  const bool two = !bwd_lean(S, KC, true, true) &&
+                   (bwd_two_pass(S, KC, false, true) || bwd_two_pass_r(S, KC, false, true) ||
+                    bwd_two_pass_g(S, KC, true, true));
   const int act = two ? (p.activation != 0 ? 1 : 0) : 2;
   return KC * 4 + act;
 }

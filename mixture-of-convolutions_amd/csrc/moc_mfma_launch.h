@@ -194,11 +194,11 @@ constexpr bool bwd_two_pass(int S, int KC, bool act, bool bf) {
 }
 // With the activation, the two passes where the fused pass spills or forms the
 // same work per route chunk (bf16: 64 routes and 3 to 8 taps, 9 to 16 taps, and
-// of the prefill's shapes below 32 routes; measured against the fused pass): the dx
+// the prefill's 32 routes with 6 to 8 taps; measured against the fused pass): the dx
 // pass forms g = dy silu'(P) and leaves it in the workspace (fp32 [N, D]) for the
-// taps pass.  Single launches only (the grouped launch keeps the fused pass).
+// taps pass.
 constexpr bool bwd_two_pass_g(int S, int KC, bool act, bool bf) {
-  return act && ((bf && ((KC == 2 && S >= 5) || (KC == 1 && S >= 8) || (KC == 4 && S >= 3))) ||
+  return act && ((bf && ((KC == 2 && S >= 6) || (KC == 1 && S >= 9) || (KC == 4 && S >= 3))) ||
                  (!bf && f32_two_pass(S, KC)));
 }
 // The prefill runs those two passes (the dx pass's P reading the cache) with 32
