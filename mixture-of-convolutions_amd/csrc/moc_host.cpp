@@ -8,9 +8,9 @@
 // Why: a step of a small layer spent most of its time in the interpreter: checks,
 // argument conversion and allocations in Python, and a backward that waits for
 // the interpreter lock on autograd's own thread.  Us a call, Python functions ->
-// here: training step B 3 T 1021 D 1130 163 -> 93 (53 of it kernels), fp32 B 2
-// T 512 D 256 170 -> 95; 777-token prefill 30.6 -> 17.6; decode step 10.4 -> 7.1,
-// fp32 25.6 -> 11.0.
+// here: training step B 3 T 1021 D 1130 138 to 165 (by box) -> 92 (53 of it
+// kernels), fp32 B 2 T 512 D 256 170 -> 95; 777-token prefill 31 -> 17.6; decode step
+// 10.5 -> 7.6, fp32 25.6 -> 11.4.
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>

@@ -251,6 +251,10 @@ inline Grid2 bwd_taps_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int n_cu
 // them, and a grid below one round of workgroups took twice a step (bf16, 32 routes,
 // 2 taps, 2000 tokens, D 128: 63 ranges of 1 or 2 steps 15.4 us, 65 of one 12.5).
 // Every range has at least one step: there are at most ceil(N / (32 - (S - 1))).
+// The older workgroups' share, measured on this kernel (both stages, us, share 50 / 54 /
+// 58 / 62 / 66 / 70 percent): B4 T4096 D2048, 4 taps, SiLU 92 / 87 / 86 / 84 / 85 / 88,
+// without 81.5 / 79 / 78.5 / 77.5 / 79.5 / 82; 32768 packed tokens, D 4096 276 / 271 / 269 /
+// 272-277 / 282 / 285; 2 taps 72 / 75 / 75 / 71 / 72 / 75.
 inline Grid2 bwd_lean_grid(int64_t N, int64_t gx, int64_t D, int64_t S, int KC, bool bf, int n_cu) {
   const bool four = lean_waves(static_cast<int>(S), KC, bf) == 4;
   Grid2 g = four ? bwd_grid_tiered(N, gx, D, S, n_cu)
