@@ -199,8 +199,9 @@ def _moc_forward(ctx, x, alpha, basis, activation, routing, cu_seqlens, max_seql
     return y
 
 
-def _moc_backward(ctx, dy):
-    saved = ctx.saved_tensors
+def _moc_backward(ctx, saved, dy):
+    """``saved``: ctx.saved_tensors, unpacked once (a checkpoint's hooks allow
+    no second time)."""
     x, alpha, basis = saved[:3]
     cu_seqlens = saved[3 + ctx.n_extra] if ctx.varlen else None
     return ops.launch_backward(x, alpha, basis, dy, activation_flag=ctx.act,
@@ -220,7 +221,7 @@ class _MoCFunction(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, dy):
-        dx, dalpha, dbasis = _moc_backward(ctx, dy)
+        dx, dalpha, dbasis = _moc_backward(ctx, ctx.saved_tensors, dy)
         return dx, dalpha, dbasis, None, None, None, None, None
 
 
@@ -237,7 +238,7 @@ class _MoCRoutedFunction(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, dy):
-        dx, dlogits, dbasis = _moc_backward(ctx, dy)
+        dx, dlogits, dbasis = _moc_backward(ctx, ctx.saved_tensors, dy)
         return dx, dlogits, dbasis, None, None, None, None, None, None
 
 
@@ -277,8 +278,9 @@ class _MoCLayerFunction(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, dy):
-        dx, dlogits, dbasis = _moc_backward(ctx, dy)
-        z, router = ctx.saved_tensors[3:5]
+        saved = ctx.saved_tensors
+        dx, dlogits, dbasis = _moc_backward(ctx, saved, dy)
+        z, router = saved[3:5]
         dz = dr = None
         if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
             dz, dr = ops.router_backward(z, router, dlogits, ctx.needs_input_grad[1],

@@ -10,6 +10,7 @@ import time
 import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
+from torch.utils.checkpoint import checkpoint
 
 import moc
 from moc import MoC, api
@@ -131,6 +132,29 @@ def test_autograd_promises():
         z.add_(1)
     with pytest.raises(RuntimeError, match="inplace"):
         torch.autograd.grad(y, [x], torch.ones_like(y))
+
+
+@pytest.mark.parametrize("dtype", [BF, F32])
+def test_checkpointed_layer(dtype):
+    """A checkpoint's saved tensors are unpacked once: the nodes of the host module
+    and of the Python functions."""
+    m, g = _layer(dtype), gen(13)
+    x, z = (randn(g, 2, 20, n).to(DEV, dtype).requires_grad_() for n in (130, 128))
+    cu = torch.tensor([0, 20, 40], dtype=torch.int32)
+    xp, zp = x.detach().flatten(0, 1).requires_grad_(), z.detach().flatten(0, 1).requires_grad_()
+    dy = randn(g, 2, 20, 130).to(DEV, dtype)
+    want = torch.autograd.grad(m(x, z)[0], [x, z], dy)
+    calls = {"host": (lambda a, b: m(a, b)[0], x, z), "python": (lambda a, b: _python(m, a, b), x, z),
+             "offsets on the host": (lambda a, b: m(a, b, cu_seqlens=cu.to(DEV), max_seqlen=20, cu_seqlens_cpu=cu)[0],
+                                     xp, zp),
+             "functional": (lambda a, b: moc.moc_triton(a, b[..., :16].softmax(-1), m.conv_bases)[0], x, z)}
+    for name, (f, a, b) in calls.items():
+        d = dy.view(a.shape)
+        got = torch.autograd.grad(checkpoint(f, a, b, use_reentrant=False), [a, b], d)
+        ref = torch.autograd.grad(f(a, b), [a, b], d)
+        assert all(torch.equal(u, v) for u, v in zip(got, ref)), name
+        if name != "functional":
+            assert all(torch.equal(u.view_as(v), v) for u, v in zip(got, want)), name
 
 
 def test_watched_calls_stay_with_python():
