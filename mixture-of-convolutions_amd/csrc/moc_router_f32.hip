@@ -13,7 +13,7 @@
 // K % 4 == 0, K <= 32, Z % 64 == 0.
 
 #include "moc_kernels.h"
-#include "moc_mfma.h"
+#include "moc_mfma_launch.h"
 
 namespace moc {
 namespace router {
@@ -320,11 +320,12 @@ void router_f32_forward(const void* z, const void* r, void* out, int64_t N, int6
   // Z 512, 16384 tokens: 13.9 and 12.1; below Z 512 four waves' shorter sums are 20%
   // closer to 64 bits for 0.4 us)
   const int64_t blocks = router::cdiv(N, 16);
-  const bool eight = blocks <= 256 && Z >= 512;
+  const int n_cu = mfma::device_cu_count(), cus = n_cu > 0 ? n_cu : 256;
+  const bool eight = blocks <= cus && Z >= 512;
   // more than 16 routes in two workgroups of 16 where half the CUs would be idle and
   // no softmax joins them: a CU's matrix rate bounds a token block (decode step of 16
   // tokens, Z 4096, 32 routes: its router 12.8 -> 8.0 us)
-  const bool halves = K > 16 && routing != ROUTE_SOFTMAX && 2 * blocks <= 256;
+  const bool halves = K > 16 && routing != ROUTE_SOFTMAX && 2 * blocks <= cus;
   const bool one = K <= 16 || halves;
   auto kern = one ? (eight ? router::router_f32_fwd_kernel<1, 8> : router::router_f32_fwd_kernel<1, 4>)
                   : (eight ? router::router_f32_fwd_kernel<2, 8> : router::router_f32_fwd_kernel<2, 4>);

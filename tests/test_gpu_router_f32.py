@@ -44,8 +44,8 @@ def test_router_f32_edges(N, Z, K):
     assert torch.equal(ops.router_backward(z, r, dl, False, True)[1], dr)
 
 
-# each workgroup form of the forward at its first and last token count: eight waves up to
-# 256 blocks of 16 tokens from Z 512, routes past 16 halved (no softmax) up to 128 blocks
+# each workgroup form of the forward at its first and last token count (256 CUs): eight waves
+# up to 256 blocks of 16 tokens from Z 512, routes past 16 halved (no softmax) up to 128 blocks
 @pytest.mark.parametrize("N,Z,K", [(4096, 512, 16), (4097, 512, 20), (4096, 448, 4), (2048, 512, 28), (2049, 576, 32),
                                    (5, 1088, 24), (1, 4096, 32), (33, 64, 20)])
 def test_router_f32_workgroup_forms(N, Z, K):
